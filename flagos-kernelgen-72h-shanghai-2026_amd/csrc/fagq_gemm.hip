@@ -7,8 +7,9 @@
 // src/task01_fused_add_rmsnorm_group_quant.py:1731-1851, stops at the
 // quantized tensor and scales); this is the layer those formats feed.
 //
-// Work mapping.  A workgroup computes a 256 x BN tile of C (BN = 256, or 192
-// where that suits N): 8 waves of 64 x BN / 2 for every scale format, each
+// Work mapping of large products (small ones, whose 256-row tiles would leave
+// CUs idle, take the tiles of fagq_gemm_small.hpp).  A workgroup computes a
+// 256 x BN tile of C (BN = 256, or 192 where that suits N): 8 waves of 64 x BN / 2 for every scale format, each
 // wave a grid of 16 x 16 tiles, each one v_mfma_scale_f32_16x16x128_f8f6f4
 // per 128-deep k-block.  The weight tile is the MFMA's first operand and the activation
 // tile its second, so each lane's four results are four consecutive columns
@@ -28,7 +29,8 @@
 // measures the fragment read with this f at 4 cycles per instruction and with
 // f(r) = (r >> 1) & 7 or r & 7 at 8 (a 2-way conflict on every read).
 //
-// Pipeline (fagq_gemm_pp_kernel).  Five 32 KB slots, all 160 KB of LDS,
+// Pipeline of large products (fagq_gemm_pp_kernel; the others are in
+// fagq_gemm_small.hpp).  Five 32 KB slots, all 160 KB of LDS,
 // hold the tile sequence A(0), B(0), A(1), B(1), ...; the 8 waves are two
 // groups of four half a k-block apart, so that one group's products run
 // while the other reads its fragments from LDS and issues the copies.
@@ -45,6 +47,8 @@
 // 0, so a 16-column tile is wholly inside or outside).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "fagq.h"
 #include "fagq_diag.h"
@@ -114,17 +118,18 @@ struct GArgs {
 };
 
 // Workgroup b runs on XCD b % 8.  XCD x takes one contiguous range of the
-// tile order, and the order walks kGroupM row tiles at a time column by
+// tile order, and the order walks group_m row tiles at a time column by
 // column, so the tiles an XCD has in flight share a few row and column
 // panels in its L2.
-__device__ __forceinline__ void tile_coords(int b, int m_tiles, int n_tiles, int& mt, int& nt) {
+__device__ __forceinline__ void tile_coords(int b, int m_tiles, int n_tiles, int group_m, int& mt,
+                                            int& nt) {
   const int T = m_tiles * n_tiles;
   const int x = b & 7, i = b >> 3, per = T >> 3, rem = T & 7;
   const int t = x * per + (x < rem ? x : rem) + i;
-  const int group = t / (kGroupM * n_tiles);
-  const int first_m = group * kGroupM;
-  const int gm = m_tiles - first_m < kGroupM ? m_tiles - first_m : kGroupM;
-  const int w = t - group * kGroupM * n_tiles;
+  const int group = t / (group_m * n_tiles);
+  const int first_m = group * group_m;
+  const int gm = m_tiles - first_m < group_m ? m_tiles - first_m : group_m;
+  const int w = t - group * group_m * n_tiles;
   mt = first_m + w % gm;
   nt = w / gm;
 }
@@ -169,7 +174,74 @@ __device__ __forceinline__ void pp_barrier() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// The GEMM kernel: the ping-pong pipeline.  The 8 waves form two groups of
+// One scale at byte offset `off`, as loaded (fp32 bits or the UE8M0 byte).
+template <int SF>
+__device__ __forceinline__ uint32_t load_scale(const rsrc_t& rs, uint32_t off) {
+  if constexpr (SF == SF_F32) return __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0);
+  else return (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(rs, off, 0, 0);
+}
+template <int SF>
+__device__ __forceinline__ float scale_value(uint32_t s) {
+  return SF == SF_UE8M0 ? e8m0_to_f32(s) : __uint_as_float(s);
+}
+
+// One k-block's products of TN x TM tiles: weight fragments bf with scale sb,
+// activation fragments af with the lane's row scales sa.  Both UE8M0: the
+// matrix core applies the scales; else each product goes to a temporary and is
+// added as fmaf(t, sa * sb, acc).
+template <int ASF, int BSF, int TM, int TN>
+__device__ __forceinline__ void products(f32x4 (&acc)[TN][TM], const i32x8 (&bf)[TN],
+                                         const i32x8 (&af)[TM], uint32_t sb,
+                                         const uint32_t (&sa)[TM]) {
+  if constexpr (ASF == SF_UE8M0 && BSF == SF_UE8M0) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int t = 0; t < TM; ++t)
+        acc[j][t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+            bf[j], af[t], acc[j][t], 0, 0, 0, (int)sb, 0, (int)sa[t]);
+  } else {
+    float sm[TM];
+#pragma unroll
+    for (int t = 0; t < TM; ++t) sm[t] = scale_value<ASF>(sa[t]) * scale_value<BSF>(sb);
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int t = 0; t < TM; ++t) {
+        const f32x4 p = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+            bf[j], af[t], f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0, 127, 0, 127);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[j][t][e] = __builtin_fmaf(p[e], sm[t], acc[j][t][e]);
+      }
+  }
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int t = 0; t < TM; ++t) pin(acc[j][t]);
+}
+
+// A lane's four outputs of a 16 x 16 tile: row `row` of the buffer, columns
+// ncol + 4 (lane / 16) .. + 3.  Rows past the buffer are dropped.
+__device__ __forceinline__ void store_tile(const rsrc_t& rc, int N, const f32x4& acc, int row,
+                                           int ncol, int lane) {
+  const u32x2 v = {pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3])};
+  const uint32_t off =
+      ((uint32_t)row * (uint32_t)N + (uint32_t)(ncol + 4 * (lane >> 4))) * 2u;
+  __builtin_amdgcn_raw_buffer_store_b64(v, rc, off, 0, 0);
+}
+
+// f(integral_constant<int, 0>) .. f(integral_constant<int, N - 1>), in order.
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void unrolled(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>());
+    unrolled<N, I + 1>(f);
+  }
+}
+
+#include "fagq_gemm_small.hpp"
+
+// The kernel for large products: the ping-pong pipeline.  The 8 waves form two groups of
 // 4: group 0 (waves 0-3) owns the tile's columns 0 .. BN / 2 - 1, group 1
 // (waves 4-7) the other half, and each SIMD runs one wave of each.  Every
 // k-block spans two barrier intervals, and group 1 runs half a k-block
@@ -211,7 +283,7 @@ __global__ void __launch_bounds__(L::THREADS, 1) fagq_gemm_pp_kernel(const GArgs
   const int wm = wave % L::WAVES_M, wn = wave / L::WAVES_M;
   const bool g0 = wn == 0;
   int mt, nt;
-  tile_coords((int)blockIdx.x, g.m_tiles, g.n_tiles, mt, nt);
+  tile_coords((int)blockIdx.x, g.m_tiles, g.n_tiles, kGroupM, mt, nt);
   const int m0 = mt * kBM, n0 = nt * L::BN;
   const int mrows = g.M - m0 < kBM ? g.M - m0 : kBM;
   const int nrows = g.N - n0 < L::BN ? g.N - n0 : L::BN;
@@ -411,14 +483,7 @@ __global__ void __launch_bounds__(L::THREADS, 1) fagq_gemm_pp_kernel(const GArgs
     const int ncol = wcol + 16 * j;
     if (ncol >= g.N) continue;   // uniform over the wave
 #pragma unroll
-    for (int i = 0; i < kTM; ++i) {
-      const uint32_t row = (uint32_t)(wm * 16 * kTM + 16 * i + (lane & 15));
-      u32x2 v;
-      v[0] = pack_bf16x2(acc[j][i][0], acc[j][i][1]);
-      v[1] = pack_bf16x2(acc[j][i][2], acc[j][i][3]);
-      const uint32_t off = (row * (uint32_t)g.N + (uint32_t)(ncol + 4 * (lane >> 4))) * 2u;
-      __builtin_amdgcn_raw_buffer_store_b64(v, rc, off, 0, 0);
-    }
+    for (int i = 0; i < kTM; ++i) store_tile(rc, g.N, acc[j][i], wm * 16 * kTM + 16 * i + (lane & 15), ncol, lane);
   }
 }
 
@@ -478,13 +543,99 @@ int pick_bn(int64_t M, int64_t N) {
   return cost(Layout192::BN) < cost(Layout256::BN) ? Layout192::BN : Layout256::BN;
 }
 
+// The tiles for small products (fagq_gemm_small.hpp), each with its cost model:
+// us = c0 + nk t0 for up to one tile per CU, and c1 + nk t1 for each further
+// round of 256, nk = K / 128.  Least-squares fits of the relative error over M 1 .. 4096, N
+// 256 .. 4096, K 512 .. 7168 with fp32 and UE8M0 scales (MI355X, 384 shapes, replayed graphs,
+// operands rotated): 80 % of the points within 15 %, and the choice by these
+// numbers took 0.6 % longer than the fastest tile of each shape (geometric mean),
+// 11 % at worst.
+enum SmallTile { kWaves16x16, kWaves32x32, kWaves32x64, kRing64x64, kRing128x64, kRing128x128,
+                 kRing192x128, kNumSmall, kNoSmall = -1 };
+struct SmallInfo {
+  int bm, bn, threads;
+  double c0, t0, c1, t1;
+};
+constexpr SmallInfo kSmall[kNumSmall] = {
+    {16, 16, 512, 2.76, 0.043, 0.27, 0.045},  {32, 32, 512, 2.97, 0.078, 0.60, 0.098},
+    {32, 64, 512, 3.46, 0.124, 2.04, 0.150},  {64, 64, 256, 3.26, 0.233, 1.36, 0.170},
+    {128, 64, 512, 3.63, 0.334, 2.02, 0.281}, {128, 128, 512, 4.73, 0.490, 4.03, 0.569},
+    {192, 128, 512, 6.35, 0.673, 6.12, 0.779}};
+using Ring64x64 = Ring<2, 2, 2, 2, 5>;       // two workgroups per CU
+using Ring128x64 = Ring<2, 2, 4, 2, 3>;      // two workgroups per CU
+using Ring128x128 = Ring<2, 4, 4, 2, 3>;
+using Ring192x128 = Ring<3, 4, 4, 2, 4>;
+// The same for one round of 256-row tiles, 256 and 192 columns wide.
+constexpr double kPP256C = 13.0, kPP256T = 1.368, kPP192C = 6.87, kPP192T = 0.923;
+constexpr int64_t kSmallMinBlocks = 4;       // k-blocks: the fits' range ends at K = 512
+constexpr int64_t kSmallMaxK = 1 << 16;      // row offsets of 192 rows stay far below 2^31
+constexpr int64_t kSmallMaxRows = 1 << 16;   // M and N of a forced small tile: a call's own reach
+
+// The small tile for a product, or kNoSmall where the 256-row tiles stay:
+// where these fill the chip once and more, outside the fits' range of K, and
+// unless a small tile is 5 % faster by the model (the model's own error).
+int pick_small(int64_t M, int64_t N, int64_t K, int pp_bn) {
+  const int64_t nk = K / kBK;
+  if (nk < kSmallMinBlocks || K > kSmallMaxK ||
+      ceil_div(M, kBM) * ceil_div(N, pp_bn) > kCUs)
+    return kNoSmall;
+  double best = 0.95 * (pp_bn == Layout192::BN ? kPP192C + kPP192T * (double)nk
+                                               : kPP256C + kPP256T * (double)nk);
+  int pick = kNoSmall;
+  for (int i = 0; i < kNumSmall; ++i) {
+    const SmallInfo& t = kSmall[i];
+    const int64_t rounds = ceil_div(ceil_div(M, t.bm) * ceil_div(N, t.bn), kCUs);
+    const double us = t.c0 + t.t0 * (double)nk + (double)(rounds - 1) * (t.c1 + t.t1 * (double)nk);
+    if (us < best) {
+      best = us;
+      pick = i;
+    }
+  }
+  return pick;
+}
+
+template <int ASF, int BSF>
+const void* small_kernel(int tile) {
+  switch (tile) {
+    case kWaves16x16:
+      return reinterpret_cast<const void*>(&fagq_gemm_waves_kernel<ASF, BSF, 1, 1, 8, 2>);
+    case kWaves32x32:
+      return reinterpret_cast<const void*>(&fagq_gemm_waves_kernel<ASF, BSF, 2, 2, 8, 1>);
+    case kWaves32x64:
+      return reinterpret_cast<const void*>(&fagq_gemm_waves_kernel<ASF, BSF, 2, 4, 8, 1>);
+    case kRing64x64:
+      return reinterpret_cast<const void*>(&fagq_gemm_ring_kernel<ASF, BSF, Ring64x64>);
+    case kRing128x64:
+      return reinterpret_cast<const void*>(&fagq_gemm_ring_kernel<ASF, BSF, Ring128x64>);
+    case kRing128x128:
+      return reinterpret_cast<const void*>(&fagq_gemm_ring_kernel<ASF, BSF, Ring128x128>);
+    default:
+      return reinterpret_cast<const void*>(&fagq_gemm_ring_kernel<ASF, BSF, Ring192x128>);
+  }
+}
+const void* small_kernel_for(int tile, int asf, int bsf) {
+  const bool au = asf == FAGQ_SCALE_UE8M0, bu = bsf == FAGQ_SCALE_UE8M0;
+  if (au) return bu ? small_kernel<SF_UE8M0, SF_UE8M0>(tile) : small_kernel<SF_UE8M0, SF_F32>(tile);
+  return bu ? small_kernel<SF_F32, SF_UE8M0>(tile) : small_kernel<SF_F32, SF_F32>(tile);
+}
+
+// `bn`: 0 for the shape's own kernel and tile; 192 or 256 for that width of the
+// 256-row tiles; 1 + i for small tile i.
 int launch(const void* a_q, const void* a_scale, const void* b_q, const void* b_scale, void* c,
            int64_t M, int64_t N, int64_t K, int asf, int asl, int bsf, int bn, void* stream) {
   const int v = validate(a_q, a_scale, b_q, b_scale, c, M, N, K, asf, asl, bsf);
   if (v != FAGQ_OK || M == 0) return v;
   const int dc = device_check();
   if (dc != FAGQ_OK) return dc;
-  if (bn == 0) bn = pick_bn(M, N);
+  int small = kNoSmall;
+  if (bn == 0) {
+    bn = pick_bn(M, N);
+    small = pick_small(M, N, K, bn);
+  } else if (bn <= kNumSmall) {
+    small = bn - 1;
+  }
+  const int bm = small == kNoSmall ? kBM : kSmall[small].bm;
+  if (small != kNoSmall) bn = kSmall[small].bn;
   GArgs g;
   g.a = static_cast<const uint8_t*>(a_q);
   g.as = static_cast<const uint8_t*>(a_scale);
@@ -498,16 +649,17 @@ int launch(const void* a_q, const void* a_scale, const void* b_q, const void* b_
   const bool col = asl == FAGQ_LAYOUT_COL_MAJOR;
   g.as_kstride = col ? (int32_t)M : 1;
   g.as_mstride = col ? 1 : g.kblocks;
-  g.m_tiles = (int32_t)ceil_div(M, kBM);
+  g.m_tiles = (int32_t)ceil_div(M, bm);
   g.n_tiles = (int32_t)ceil_div(N, bn);
   g.as_bytes = (uint32_t)(M * g.kblocks * (asf == FAGQ_SCALE_F32 ? 4 : 1));
   g.bs_bytes = (uint32_t)(ceil_div(N, 128) * g.kblocks * (bsf == FAGQ_SCALE_F32 ? 4 : 1));
   void* args[] = {&g};
-  const void* kernel = bn == Layout192::BN ? kernel_for_layout<Layout192>(asf, bsf)
-                                           : kernel_for_layout<Layout256>(asf, bsf);
-  return launch_kernel(kernel, dim3((unsigned)(g.m_tiles * g.n_tiles)),
-                       dim3((unsigned)Layout256::THREADS), args, 0,
-                       static_cast<hipStream_t>(stream));
+  const void* kernel = small != kNoSmall     ? small_kernel_for(small, asf, bsf)
+                       : bn == Layout192::BN ? kernel_for_layout<Layout192>(asf, bsf)
+                                             : kernel_for_layout<Layout256>(asf, bsf);
+  const int threads = small != kNoSmall ? kSmall[small].threads : Layout256::THREADS;
+  return launch_kernel(kernel, dim3((unsigned)(g.m_tiles * g.n_tiles)), dim3((unsigned)threads),
+                       args, 0, static_cast<hipStream_t>(stream));
 }
 
 }  // namespace
@@ -531,7 +683,12 @@ FAGQ_API int fagq_gemm_launch_mapped(const void* a_q, const void* a_scale, const
                                      const void* b_scale, void* c, int64_t M, int64_t N,
                                      int64_t K, int a_scale_format, int a_scale_layout,
                                      int b_scale_format, int block_n, void* stream) {
-  if (block_n != 0 && block_n != Layout192::BN && block_n != Layout256::BN) return FAGQ_E_FORMAT;
+  const bool small = block_n > 0 && block_n <= kNumSmall;
+  if (!small && block_n != 0 && block_n != Layout192::BN && block_n != Layout256::BN)
+    return FAGQ_E_FORMAT;
+  // A forced small tile: K and the number of workgroups within what it takes.
+  if (small && K > 0 && (K > kSmallMaxK || M > kSmallMaxRows || N > kSmallMaxRows))
+    return FAGQ_E_TOO_LARGE;
   return launch(a_q, a_scale, b_q, b_scale, c, M, N, K, a_scale_format, a_scale_layout,
                 b_scale_format, block_n, stream);
 }
@@ -540,11 +697,14 @@ FAGQ_API int fagq_gemm_query_route(int64_t M, int64_t N, int64_t K, fagq_gemm_ro
   if (!route) return FAGQ_E_NULL;
   if (M < 0 || N <= 0 || K <= 0 || N % 16 != 0 || K % kBK != 0) return FAGQ_E_SHAPE;
   const int bn = pick_bn(M, N);
-  route->block_m = kBM;
-  route->block_n = bn;
-  route->block_threads = Layout256::THREADS;
-  route->group_m = kGroupM;
-  route->grid_blocks = ceil_div(M, kBM) * ceil_div(N, bn);
+  const int small = pick_small(M, N, K, bn);
+  const int64_t bm = small == kNoSmall ? kBM : kSmall[small].bm;
+  route->block_m = (int32_t)bm;
+  route->block_n = small == kNoSmall ? bn : kSmall[small].bn;
+  route->block_threads = small == kNoSmall ? Layout256::THREADS : kSmall[small].threads;
+  // The waves kernels walk all row tiles of a column tile before the next.
+  route->group_m = small == kNoSmall || small >= kRing64x64 ? kGroupM : (int32_t)ceil_div(M, bm);
+  route->grid_blocks = ceil_div(M, bm) * ceil_div(N, route->block_n);
   return FAGQ_OK;
 }
 

@@ -17,8 +17,11 @@
  * quantized tensor and its scales; this is the consumer of that wire format.
  *
  * Accumulation is fp32 inside each 128-deep block (the MFMA's own order),
- * then fp32 across blocks in block order.  With both scales UE8M0 the scales
- * are applied by the matrix core itself (exact powers of two).
+ * then fp32 across blocks: in block order, or for small products (tiles of
+ * 16 x 16 to 32 x 64, fagq_gemm_query_route) in eight interleaved partial sums
+ * that are then added.  The order depends on the shape alone, so equal calls
+ * give equal bits.  With both scales UE8M0 the scales are applied by the matrix
+ * core itself (exact powers of two).
  *
  * Same conventions as fagq.h: device pointers, stream-ordered, no allocation,
  * no synchronization; returns 0, a FAGQ_E_* code (> 0) or -hipError_t.
