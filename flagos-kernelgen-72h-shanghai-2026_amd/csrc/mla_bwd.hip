@@ -8,19 +8,14 @@
 //   rows i >= E: dq_i = scale * do_i
 //   dc_j = sum_{i >= j} hs_i / (i + 1), hs_i = sum_h do[h, i]
 //
-// Kernels, in stream order:
+// Kernels, in stream order.  Long sequences (see is_short):
 //   K1 mla_stream_do   - the one pass over dO (all the HBM traffic): per row
 //                        and all H heads, dq = scale * do (rows >= E) and the
 //                        head sum, stored as hs_i / (i + 1) in the workspace.
 //                        A lane owns 8 consecutive dims (16-byte loads), a
 //                        workgroup 2048 / D rows, so each head contributes a
 //                        contiguous 4 KB (D = 512) segment per workgroup.
-//                        Short sequences split the heads into up to 8 groups,
-//                        each writing a partial head-sum plane.
-//   K2 mla_block_totals - per block of 16-64 rows (or column slice of one):
-//                        fp32 totals of hs / (i + 1) over rows and head-group
-//                        planes; each row's plane sum is written back over
-//                        plane 0.
+//   K2 mla_block_totals - per block of 16-64 rows: fp32 totals of hs / (i + 1).
 //   K3 mla_exact_rows_suffix_scan - one launch of 1024-thread workgroups, two
 //                        kinds:
 //                        * exact rows, one per (b, h): q, do and c rows 0..E-1
@@ -29,13 +24,15 @@
 //                          where the reference rounds, dq rows 0..E-1 (which
 //                          K1 does not write);
 //                        * per block: carry = totals of all later blocks, then
-//                          the reverse running sum over the block's rows
-//                          (plane 0), written as dc.
+//                          the reverse running sum over the block's rows,
+//                          written as dc.
 //                        The exact rows depend on nothing K1 or K2 writes;
 //                        sharing the last launch with the few scan workgroups
 //                        runs them in the part of the chip those leave idle.
 // K2 and K3 issue each thread's loads as one batch: at these sizes they are
 // latency-bound: every dependent round trip to memory adds its full latency.
+// Short sequences, two launches: mla_short_do (the dO pass with the running
+// sums of 8-row blocks, and the exact rows) and mla_short_scan.
 //
 // D above kSliceD (512) runs as column slices of at most kSliceD dims: K1, the
 // block totals and K3 are per column, so each slice runs them on its columns
@@ -71,13 +68,11 @@ struct MArgs {
   const float* lse;
   void* dq;
   void* dc;
-  float* hs;          // workspace: [hsplit, B, S, D] partial head sums / (i + 1)
+  float* hs;          // workspace: [B, S, D] head sums / (i + 1); for short sequences their
+                      // reverse running sums within blocks of kBlockRows rows
   float* tot;         // workspace: [B, nblk, D] block totals
-  int64_t hs_split;   // elements between the partial head-sum planes (B * S * D)
   int32_t brows;      // rows per scan block
   int32_t nblk;       // ceil(S / brows)
-  int32_t hsplit;     // head groups K1 splits the heads into
-  int32_t hps;        // heads per group
   int32_t H, S;
   int32_t D;          // dims of this column slice (the width K1, K2 and K3's scan handle)
   int32_t ld;         // elements between rows of q, c, out, dout, dq and dc (the full D);
@@ -87,8 +82,6 @@ struct MArgs {
   float scale;
   int32_t dq_bf16;    // dq is bf16 (else fp32)
   int32_t dc_bf16;
-  int32_t bsplit_sh;  // K2 workgroups per scan block = 1 << bsplit_sh, each summing
-                      // D >> bsplit_sh of its columns
 };
 
 __device__ __forceinline__ float bf16_to_f(uint32_t h) { return __uint_as_float(h << 16); }
@@ -113,28 +106,34 @@ __device__ __forceinline__ void store8(const rsrc_t& rs, bool bf16, uint32_t e, 
   }
 }
 
-// ------------------------------------------------------------------ K1
+// ------------------------------------------------------------------ the dO pass
 
-// grid (ceil(S / rows_per_wg), B, hsplit); rows_per_wg = 256 / (D / 8);
-// z picks the head group [z hps, min(H, (z + 1) hps)).  U heads' loads are in
-// flight per lane: for grids of 2048 and more U = 2 with bf16 dq (50 VGPRs, 8
-// workgroups per CU) and U = 1 with fp32 dq, whose stores are twice the
-// loads' bytes (2 B / 4 B, 2 x 64 x 4096 x 512: 297 against 308 us for the
-// pass); U = 8 (110 VGPRs, 4 per CU) for grids that fit 4 per CU, where each
-// workgroup's few heads are then loaded at once.
+// 8 fp32 values of a lane: one 16-byte bf16 or two 16-byte fp32 stores at
+// element xa (HALVES: fp32, the second at xb).
+template <bool HALVES>
+__device__ __forceinline__ void store_lane(const rsrc_t& rs, bool bf16, uint32_t xa, uint32_t xb,
+                                           const float (&v)[8]) {
+  if constexpr (HALVES) {
+    const u32x4 x = {__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]),
+                     __float_as_uint(v[3])};
+    const u32x4 y = {__float_as_uint(v[4]), __float_as_uint(v[5]), __float_as_uint(v[6]),
+                     __float_as_uint(v[7])};
+    __builtin_amdgcn_raw_buffer_store_b128(x, rs, xa * 4u, 0, kNonTemporal);
+    __builtin_amdgcn_raw_buffer_store_b128(y, rs, xb * 4u, 0, kNonTemporal);
+  } else {
+    store8(rs, bf16, xa, v);
+  }
+}
+
+// A lane's 8 elements of one row over heads hbeg .. hend - 1 of batch b: dq =
+// scale * dO (rows >= E) and their sum, acc.  The elements are 8 consecutive
+// from ea (of head 0), or with HALVES 4 from ea and 4 from eb.  Heads in
+// batches of U, software-pipelined: the loads of batch i + 1 are issued before
+// batch i is consumed.  Heads past hend re-read head hend - 1 (in bounds) and
+// are not used.
 template <int U, bool HALVES>
-__global__ void __launch_bounds__(kThreads) mla_stream_do(const MArgs g) {
-  const int lpr = g.D / 8;                        // lanes per row
-  const int t = threadIdx.x;
-  // When lpr does not divide kThreads, the last kThreads % lpr threads hold
-  // no whole row of this workgroup (their t / lpr would be the next
-  // workgroup's first row), and stop here.
-  if (t / lpr >= kThreads / lpr) return;
-  const int row = (int)blockIdx.x * (kThreads / lpr) + t / lpr;
-  if (row >= g.S) return;
-  const int b = (int)blockIdx.y;
-  const int hbeg = (int)blockIdx.z * g.hps;
-  const int hend = hbeg + g.hps < g.H ? hbeg + g.hps : g.H;
+__device__ __forceinline__ void stream_heads(const MArgs& g, int b, int row, uint32_t ea,
+                                             uint32_t eb, int hbeg, int hend, float (&acc)[8]) {
   const uint32_t hsd = (uint32_t)g.H * (uint32_t)g.S * (uint32_t)g.ld;   // elements per batch
   // The slice's elements of batch b end at (H S - 1) ld + D (the descriptors'
   // size, so they stay inside the tensors whatever the slice's first column).
@@ -142,23 +141,9 @@ __global__ void __launch_bounds__(kThreads) mla_stream_do(const MArgs g) {
   const rsrc_t rdo = make_rsrc(g.dout + (int64_t)b * hsd, span * 2u);
   const rsrc_t rdq = make_rsrc((const uint8_t*)g.dq + (int64_t)b * hsd * (g.dq_bf16 ? 2 : 4),
                                span * (g.dq_bf16 ? 2u : 4u));
-  // Elements of the lane (head 0): 8 consecutive from ea, or with HALVES 4
-  // from ea and 4 from eb = ea + D / 2, so that each of its two 16-byte fp32
-  // stores lies in a contiguous half-row span of the row's lanes.  wa / wb:
-  // the same elements in the workspace's head-sum plane, rows of D.
-  const uint32_t li = (uint32_t)(t % lpr);
-  const uint32_t lo = li * (HALVES ? 4u : 8u);
-  const uint32_t ea = (uint32_t)row * (uint32_t)g.ld + lo;
-  const uint32_t eb = ea + (uint32_t)g.D / 2u;
-  const uint32_t wa = (uint32_t)row * (uint32_t)g.D + lo;
-  const uint32_t wb = wa + (uint32_t)g.D / 2u;
   const uint32_t hstride = (uint32_t)g.S * (uint32_t)g.ld;
   const bool write_dq = row >= g.erows;
   const bool dq_bf16 = g.dq_bf16 != 0;
-  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  // Heads in batches of U, software-pipelined: the loads of batch i + 1 are
-  // issued before batch i is consumed.  Heads past hend re-read head hend - 1
-  // (in bounds) and are not used.
   auto load_batch = [&](int h0, u32x4 (&v)[U]) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -171,20 +156,6 @@ __global__ void __launch_bounds__(kThreads) mla_stream_do(const MArgs g) {
       } else {
         v[u] = __builtin_amdgcn_raw_buffer_load_b128(rdo, (ea + ho) * 2u, 0, kNonTemporal);
       }
-    }
-  };
-  // 8 fp32 values of the lane: one 16-byte bf16 or two 16-byte fp32 stores at
-  // element xa (HALVES: the second at xb).
-  auto store_lane = [&](const rsrc_t& rs, bool bf16, uint32_t xa, uint32_t xb, const float (&v)[8]) {
-    if constexpr (HALVES) {
-      const u32x4 x = {__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]),
-                       __float_as_uint(v[3])};
-      const u32x4 y = {__float_as_uint(v[4]), __float_as_uint(v[5]), __float_as_uint(v[6]),
-                       __float_as_uint(v[7])};
-      __builtin_amdgcn_raw_buffer_store_b128(x, rs, xa * 4u, 0, kNonTemporal);
-      __builtin_amdgcn_raw_buffer_store_b128(y, rs, xb * 4u, 0, kNonTemporal);
-    } else {
-      store8(rs, bf16, xa, v);
     }
   };
   u32x4 cur[U], nxt[U];
@@ -207,36 +178,67 @@ __global__ void __launch_bounds__(kThreads) mla_stream_do(const MArgs g) {
 #pragma unroll
           for (int k = 0; k < 8; ++k) d[k] = f[k] * g.scale;
           const uint32_t ho = (uint32_t)(h0 + u) * hstride;
-          store_lane(rdq, dq_bf16, ea + ho, eb + ho, d);
+          store_lane<HALVES>(rdq, dq_bf16, ea + ho, eb + ho, d);
         }
       }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) cur[u] = nxt[u];
   }
+}
+
+// K1.  grid (ceil(S / rows_per_wg), B); rows_per_wg = 256 / (D / 8).  U heads'
+// loads are in flight per lane: U = 2 with bf16 dq (50 VGPRs, 8 workgroups per
+// CU) and U = 1 with fp32 dq, whose stores are twice the loads' bytes (2 B / 4
+// B, 2 x 64 x 4096 x 512: 297 against 308 us for the pass; 2 x 64 x 1900 x 512
+// 147.9 us per call against 157.2 with U = 8); U = 8 (110 VGPRs, 4 per CU) with
+// bf16 dq for grids that fit 4 per CU.
+template <int U, bool HALVES>
+__global__ void __launch_bounds__(kThreads) mla_stream_do(const MArgs g) {
+  const int lpr = g.D / 8;                        // lanes per row
+  const int t = threadIdx.x;
+  // When lpr does not divide kThreads, the last kThreads % lpr threads hold
+  // no whole row of this workgroup (their t / lpr would be the next
+  // workgroup's first row), and stop here.
+  if (t / lpr >= kThreads / lpr) return;
+  const int row = (int)blockIdx.x * (kThreads / lpr) + t / lpr;
+  if (row >= g.S) return;
+  const int b = (int)blockIdx.y;
+  // HALVES: eb = ea + D / 2, so that each of the lane's two 16-byte fp32
+  // stores lies in a contiguous half-row span of the row's lanes.  wa / wb:
+  // the same elements in the workspace's head sums, rows of D.
+  const uint32_t lo = (uint32_t)(t % lpr) * (HALVES ? 4u : 8u);
+  const uint32_t ea = (uint32_t)row * (uint32_t)g.ld + lo;
+  const uint32_t wa = (uint32_t)row * (uint32_t)g.D + lo;
+  const uint32_t half = (uint32_t)g.D / 2u;
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  stream_heads<U, HALVES>(g, b, row, ea, ea + half, 0, g.H, acc);
   const float n1 = (float)(row + 1);
   float o[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) o[k] = acc[k] / n1;
   const uint32_t sd = (uint32_t)g.S * (uint32_t)g.D;
-  const rsrc_t rhs = make_rsrc(g.hs + (int64_t)blockIdx.z * g.hs_split + (int64_t)b * sd, sd * 4u);
-  store_lane(rhs, false, wa, wb, o);
+  const rsrc_t rhs = make_rsrc(g.hs + (int64_t)b * sd, sd * 4u);
+  store_lane<HALVES>(rhs, false, wa, wa + half, o);
 }
 
 // ------------------------------------------------------------------ K3: exact rows
 
 constexpr int kWide = 1024;               // threads of K2 and K3 (16 waves)
 
-// Exact rows 0..E-1 of (b, h), wave m owning query row m for delta and dq;
-// wave 0 computes all 16 x 16 logits and dP with MFMAs.  The rows' D = ld
-// dims go through LDS in chunks of W = min(D, kSliceD): per chunk, every
-// global load is issued before the first LDS store (wave m loads 16-byte
-// piece `lane` of its q, do and out rows, thread t piece t % (W / 8) of c
-// row t / (W / 8)); buffer descriptors over rows 0..E-1 return zeros for the
-// rest.  The logits, dP and delta accumulate over the chunks; dS follows; then
+// Exact rows 0..E-1 of (b, h) by NW waves (16 or 8), wave m owning query rows
+// m, m + NW, .. for delta and dq; wave 0 computes all 16 x 16 logits and dP with
+// MFMAs.  The rows' D = ld dims go through LDS in chunks of W = min(D,
+// kSliceD): per chunk, every global load is issued before the first LDS store
+// (wave m loads 16-byte piece `lane` of its q, do and out rows, thread t piece
+// t % (W / 8) of c row t / (W / 8)); buffer descriptors over rows 0..E-1 return
+// zeros for the rest.  The logits, dP and delta accumulate over the chunks; dS follows; then
 // dq, chunk by chunk (c staged again when D > W).  Dynamic LDS: q, do and c
 // rows 0..15 of one chunk (padded by 16 bytes), then dS [16][16] and delta [16].
+template <int NW>
 __device__ __forceinline__ void exact_rows(const MArgs& g, int b, int h) {
+  constexpr int RPW = kE / NW;                    // query rows per wave
+  static_assert(RPW * NW == kE, "the waves share the rows evenly");
   extern __shared__ __align__(16) uint8_t smem[];
   const int D = g.ld, E = g.erows;
   const int W = D < kSliceD ? D : kSliceD;
@@ -254,12 +256,22 @@ __device__ __forceinline__ void exact_rows(const MArgs& g, int b, int h) {
   const rsrc_t rdo = make_rsrc(g.dout + qrow0, rbytes);
   const rsrc_t rout = make_rsrc(g.out + qrow0, rbytes);
   const rsrc_t rc = make_rsrc(g.c + (int64_t)b * g.S * D, rbytes);
-  // c rows 0..15 of the W-wide chunk at dim c0 (t < 16 W / 8 <= 1024).
-  auto stage_c = [&](int c0, int cpr) {
-    const int cr = t / cpr;
-    const uint32_t coff = cr < E ? (uint32_t)(cr * D + c0 + (t % cpr) * 8) * 2u : rbytes;
-    const u32x4 cv = __builtin_amdgcn_raw_buffer_load_b128(rc, coff, 0, 0);
-    if (t < kE * cpr) *reinterpret_cast<u32x4*>(cs + cr * ldl + (t % cpr) * 8) = cv;
+  // c rows 0..15 of the W-wide chunk at dim c0: 16 W / 8 <= 1024 pieces, RPW or
+  // fewer per thread.
+  auto load_c = [&](int c0, int cpr, u32x4 (&cv)[RPW]) {
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) {
+      const int e = t + i * 64 * NW, cr = e / cpr;
+      const uint32_t coff = cr < E ? (uint32_t)(cr * D + c0 + (e % cpr) * 8) * 2u : rbytes;
+      cv[i] = __builtin_amdgcn_raw_buffer_load_b128(rc, coff, 0, 0);
+    }
+  };
+  auto put_c = [&](int cpr, const u32x4 (&cv)[RPW]) {
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) {
+      const int e = t + i * 64 * NW;
+      if (e < kE * cpr) *reinterpret_cast<u32x4*>(cs + (e / cpr) * ldl + (e % cpr) * 8) = cv[i];
+    }
   };
 
   // Logits and dP of query row qm = lane % 16 with keys n = 4 (lane / 16) +
@@ -270,25 +282,36 @@ __device__ __forceinline__ void exact_rows(const MArgs& g, int b, int h) {
   // on the GPU).  Rows past E were staged as zeros.
   const int qm = lane & 15, k0 = (lane >> 4) * 8;
   f32x4 lg = {0.0f, 0.0f, 0.0f, 0.0f}, dpv = lg;
-  float delta = 0.0f;
+  float delta[RPW];
+#pragma unroll
+  for (int i = 0; i < RPW; ++i) delta[i] = 0.0f;
   for (int c0 = 0; c0 < D; c0 += W) {
     const int w = D - c0 < W ? D - c0 : W;        // a multiple of 64
     const int cpr = w / 8;                        // 16-byte pieces per row (8..64)
     if (c0 > 0) __syncthreads();                  // the previous chunk's reads are done
-    const uint32_t off = m < E && lane < cpr ? (uint32_t)(m * D + c0 + lane * 8) * 2u : rbytes;
-    const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(rq, off, 0, 0);
-    const u32x4 d = __builtin_amdgcn_raw_buffer_load_b128(rdo, off, 0, 0);
-    const u32x4 o = __builtin_amdgcn_raw_buffer_load_b128(rout, off, 0, 0);
-    stage_c(c0, cpr);
-    if (lane < cpr) {
-      *reinterpret_cast<u32x4*>(qs + m * ldl + lane * 8) = a;
-      *reinterpret_cast<u32x4*>(dos + m * ldl + lane * 8) = d;
-    }
-    // delta_m = out_m . do_m, this lane's part.
+    u32x4 a[RPW], d[RPW], o[RPW], cv[RPW];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      delta += bf16_lo(o[j]) * bf16_lo(d[j]);
-      delta += bf16_hi(o[j]) * bf16_hi(d[j]);
+    for (int i = 0; i < RPW; ++i) {
+      const int row = m + i * NW;
+      const uint32_t off = row < E && lane < cpr ? (uint32_t)(row * D + c0 + lane * 8) * 2u : rbytes;
+      a[i] = __builtin_amdgcn_raw_buffer_load_b128(rq, off, 0, 0);
+      d[i] = __builtin_amdgcn_raw_buffer_load_b128(rdo, off, 0, 0);
+      o[i] = __builtin_amdgcn_raw_buffer_load_b128(rout, off, 0, 0);
+    }
+    load_c(c0, cpr, cv);
+    put_c(cpr, cv);
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) {
+      if (lane < cpr) {
+        *reinterpret_cast<u32x4*>(qs + (m + i * NW) * ldl + lane * 8) = a[i];
+        *reinterpret_cast<u32x4*>(dos + (m + i * NW) * ldl + lane * 8) = d[i];
+      }
+      // delta_m = out_m . do_m, this lane's part.
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        delta[i] += bf16_lo(o[i][j]) * bf16_lo(d[i][j]);
+        delta[i] += bf16_hi(o[i][j]) * bf16_hi(d[i][j]);
+      }
     }
     __syncthreads();
     if (m == 0) {
@@ -308,8 +331,11 @@ __device__ __forceinline__ void exact_rows(const MArgs& g, int b, int h) {
     }
   }
 #pragma unroll
-  for (int s = 32; s > 0; s >>= 1) delta += __shfl_xor(delta, s, 64);
-  if (lane == 0) deltas[m] = delta;
+  for (int i = 0; i < RPW; ++i) {
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) delta[i] += __shfl_xor(delta[i], s, 64);
+    if (lane == 0) deltas[m + i * NW] = delta[i];
+  }
   __syncthreads();
   if (m == 0) {
     const float lse = qm < E ? g.lse[(int64_t)bh * g.S + qm] : 0.0f;
@@ -334,22 +360,27 @@ __device__ __forceinline__ void exact_rows(const MArgs& g, int b, int h) {
     const int w = D - c0 < W ? D - c0 : W;
     if (D > W) {                                  // c of this chunk (one chunk: still staged)
       __syncthreads();
-      stage_c(c0, w / 8);
+      u32x4 cv[RPW];
+      load_c(c0, w / 8, cv);
+      put_c(w / 8, cv);
       __syncthreads();
     }
-    if (m < E && lane * 8 < w) {
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) {
+      const int row = m + i * NW;
+      if (row >= E || lane * 8 >= w) continue;
       const int k = lane * 8;
       float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      for (int j = 0; j <= m; ++j) {
-        const float sv = dS[m * kE + j];
+      for (int j = 0; j <= row; ++j) {
+        const float sv = dS[row * kE + j];
         const u32x4 c = *reinterpret_cast<const u32x4*>(cs + j * ldl + k);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          acc[2 * i] = fmaf(sv, bf16_lo(c[i]), acc[2 * i]);
-          acc[2 * i + 1] = fmaf(sv, bf16_hi(c[i]), acc[2 * i + 1]);
+        for (int e = 0; e < 4; ++e) {
+          acc[2 * e] = fmaf(sv, bf16_lo(c[e]), acc[2 * e]);
+          acc[2 * e + 1] = fmaf(sv, bf16_hi(c[e]), acc[2 * e + 1]);
         }
       }
-      store8(rdq, g.dq_bf16 != 0, (uint32_t)(m * D + c0 + k), acc);
+      store8(rdq, g.dq_bf16 != 0, (uint32_t)(row * D + c0 + k), acc);
     }
   }
 }
@@ -372,82 +403,50 @@ __device__ __forceinline__ void add4(float4& a, const float4& b) {
   a.w += b.w;
 }
 
-// Thread layout of K2's block totals and K3 over D columns (K2: the
-// workgroup's column slice): cpt = D / 4 column threads (16..128) per part,
-// np = kWide / cpt parts (8..64); thread t owns columns 4 (t % cpt) .. + 3 of
-// part t / cpt (threads of parts >= np idle).
+// Thread layout of K2's block totals and K3 over D columns: cpt = D / 4 column
+// threads (16..128) per part, np = kWide / cpt parts (8..64); thread t owns
+// columns 4 (t % cpt) .. + 3 of part t / cpt (threads of parts >= np idle).
 struct Parts {
   int cpt, np, p, col;
   __device__ explicit Parts(int D) : cpt(D >> 2), np(kWide / (D >> 2)), p((int)threadIdx.x / (D >> 2)),
                                      col((int)threadIdx.x - p * (D >> 2)) {}
 };
 
-// Part p of the block's threads sums rows r0 + p, r0 + p + np, ... of the
-// block over the HS head-group planes; a batch loads all planes of
-// kBatch / HS such rows together.  With HS > 1 each row's plane sum
-// (planes in order) is written back over plane 0, so K3 reads one plane.
-// The parts' totals are joined in LDS, in part order.
-template <int HS>
-__device__ __forceinline__ void block_total_hs(const MArgs& g, int b, int blk, int cs, float4* part) {
-  constexpr int R = kBatch / HS;
-  const int cols = g.D >> g.bsplit_sh;            // this workgroup's columns: cs cols .. + cols
-  const Parts P(cols);
+// Totals of block blk (g.brows rows) of batch b: part p of the block's threads
+// sums rows r0 + p, r0 + p + np, ..., kBatch of them loaded together; the parts'
+// totals are joined in LDS, in part order.
+__device__ __forceinline__ void block_total(const MArgs& g, int b, int blk) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  float4* part = reinterpret_cast<float4*>(smem);
+  const Parts P(g.D);
   const int r0 = blk * g.brows;
   const int r1 = r0 + g.brows < g.S ? r0 + g.brows : g.S;
-  float* __restrict__ hs = g.hs + (int64_t)b * g.S * g.D + cs * cols + 4 * P.col;
+  const float* __restrict__ hs = g.hs + (int64_t)b * g.S * g.D + 4 * P.col;
   float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
   if (P.p < P.np) {
-    for (int r = r0 + P.p; r < r1; r += R * P.np) {
-      float4 v[R][HS];
+    for (int r = r0 + P.p; r < r1; r += kBatch * P.np) {
+      float4 v[kBatch];
 #pragma unroll
-      for (int i = 0; i < R; ++i) {
+      for (int i = 0; i < kBatch; ++i) {
         const int rr = r + i * P.np < r1 ? r + i * P.np : r0;
-#pragma unroll
-        for (int s = 0; s < HS; ++s)
-          v[i][s] = *reinterpret_cast<const float4*>(hs + s * g.hs_split + (int64_t)rr * g.D);
+        v[i] = *reinterpret_cast<const float4*>(hs + (int64_t)rr * g.D);
       }
 #pragma unroll
-      for (int i = 0; i < R; ++i) {
-        const int rr = r + i * P.np;
-        if (rr < r1) {
-          float4 sum = v[i][0];
-#pragma unroll
-          for (int s = 1; s < HS; ++s) add4(sum, v[i][s]);
-          if (HS > 1) *reinterpret_cast<float4*>(hs + (int64_t)rr * g.D) = sum;
-          add4(a, sum);
-        }
-      }
+      for (int i = 0; i < kBatch; ++i)
+        if (r + i * P.np < r1) add4(a, v[i]);
     }
   }
   part[threadIdx.x] = a;
   __syncthreads();
   if (P.p == 0) {
     for (int q = 1; q < P.np; ++q) add4(a, part[q * P.cpt + P.col]);
-    *reinterpret_cast<float4*>(g.tot + ((int64_t)b * g.nblk + blk) * g.D + cs * cols + 4 * P.col) = a;
+    *reinterpret_cast<float4*>(g.tot + ((int64_t)b * g.nblk + blk) * g.D + 4 * P.col) = a;
   }
 }
 
-// Totals of block blk (g.brows rows) of batch b over rows and head groups,
-// columns of slice cs (D >> bsplit_sh wide).
-__device__ __forceinline__ void block_total(const MArgs& g, int b, int blk, int cs) {
-  extern __shared__ __align__(16) uint8_t smem[];
-  float4* part = reinterpret_cast<float4*>(smem);
-  switch (g.hsplit) {                     // 1..8 (kMaxHeadSplit)
-    case 1: block_total_hs<1>(g, b, blk, cs, part); break;
-    case 2: block_total_hs<2>(g, b, blk, cs, part); break;
-    case 3: block_total_hs<3>(g, b, blk, cs, part); break;
-    case 4: block_total_hs<4>(g, b, blk, cs, part); break;
-    case 5: block_total_hs<5>(g, b, blk, cs, part); break;
-    case 6: block_total_hs<6>(g, b, blk, cs, part); break;
-    case 7: block_total_hs<7>(g, b, blk, cs, part); break;
-    default: block_total_hs<8>(g, b, blk, cs, part); break;
-  }
-}
-
-// grid (nblk << bsplit_sh, B): 1 << bsplit_sh workgroups per block.
+// grid (nblk, B)
 __global__ void __launch_bounds__(kWide) mla_block_totals(const MArgs g) {
-  const int x = (int)blockIdx.x, b = (int)blockIdx.y;
-  block_total(g, b, x >> g.bsplit_sh, x & ((1 << g.bsplit_sh) - 1));
+  block_total(g, (int)blockIdx.y, (int)blockIdx.x);
 }
 
 // ------------------------------------------------------------------ K3
@@ -525,9 +524,151 @@ __device__ __forceinline__ void suffix_scan(const MArgs& g, int b, int blk) {
 __global__ void __launch_bounds__(kWide) mla_exact_rows_suffix_scan(const MArgs g) {
   const int x = (int)blockIdx.x, b = (int)blockIdx.y;
   if (x < g.nexact)
-    exact_rows(g, b, x);
+    exact_rows<kWide / 64>(g, b, x);
   else
     suffix_scan(g, b, x - g.nexact);
+}
+
+// ------------------------------------------------------------------ short sequences
+
+// The dO pass of a short sequence.  Whole rows give few workgroups there, so a
+// workgroup takes 8 rows of a column tile of CW dims, and its 8 waves split them
+// and the heads (1 to 8 head groups): the groups' sums are joined in LDS, and
+// the block's reverse running sums (with the 1 / (i + 1)) go to the workspace,
+// whose rows 0, 8, 16, .. then are the blocks' totals.  One launch replaces a
+// pass that wrote up to 8 partial planes and a kernel for the totals, and the
+// last one only adds the later blocks' totals.  The exact rows, which depend on
+// nothing else, are the grid's first workgroups and run beside the dO pass.
+// Bound by the dO pass's bytes, and below about 20 us by the two launches'
+// latency (figures: short_tile).
+constexpr int kBlockRows = 8;
+constexpr int kShortWaves = 8;
+
+template <int CW, int U, bool HALVES>
+__global__ void __launch_bounds__(64 * kShortWaves) mla_short_do(const MArgs g) {
+  constexpr int LPR = CW / 8, WR = 64 / LPR;             // lanes per row, rows per wave
+  constexpr int RW = kBlockRows / WR, HG = kShortWaves / RW;
+  constexpr int C4 = CW / 4, T = 64 * kShortWaves;
+  static_assert(RW * WR == kBlockRows && HG * RW == kShortWaves, "waves tile the block");
+  extern __shared__ __align__(16) uint8_t smem[];        // HG x 8 x CW floats, or the exact rows'
+  const int b = (int)blockIdx.y;
+  if ((int)blockIdx.x < g.nexact) {                      // uniform over the workgroup
+    exact_rows<kShortWaves>(g, b, (int)blockIdx.x);
+    return;
+  }
+  float4* const part = reinterpret_cast<float4*>(smem);
+  const int t = threadIdx.x, lane = t & 63;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int rw = w % RW, hg = w / RW;
+  const int x = (int)blockIdx.x - g.nexact;
+  const int ncol = g.D / CW, ct = x % ncol, blk = x / ncol;   // CW divides D
+  const int r0 = blk * kBlockRows;
+  const int brow = rw * WR + lane / LPR, row = r0 + brow;     // the lane's row in the block, of S
+  const int li = lane % LPR;
+  const int hps = (g.H + HG - 1) / HG;
+  const int hbeg = hg * hps < g.H ? hg * hps : g.H;
+  const int hend = hbeg + hps < g.H ? hbeg + hps : g.H;
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (row < g.S && hbeg < hend) {
+    const uint32_t ea = (uint32_t)row * (uint32_t)g.ld + (uint32_t)(ct * CW + li * (HALVES ? 4 : 8));
+    stream_heads<U, HALVES>(g, b, row, ea, ea + CW / 2, hbeg, hend, acc);
+  }
+  float4* const mine = part + (hg * kBlockRows + brow) * C4;
+  mine[HALVES ? li : 2 * li] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  mine[HALVES ? li + C4 / 2 : 2 * li + 1] = make_float4(acc[4], acc[5], acc[6], acc[7]);
+  __syncthreads();
+  // Heads' sums in group order, into group 0's place.
+  for (int e = t; e < kBlockRows * C4; e += T) {
+    float4 v = part[e];
+#pragma unroll
+    for (int q = 1; q < HG; ++q) add4(v, part[q * kBlockRows * C4 + e]);
+    part[e] = v;
+  }
+  __syncthreads();
+  if (t < C4) {
+    float4 v[kBlockRows];
+#pragma unroll
+    for (int k = 0; k < kBlockRows; ++k) v[k] = part[k * C4 + t];
+    float* const hs = g.hs + ((int64_t)b * g.S + r0) * g.D + ct * CW + 4 * t;
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int k = kBlockRows - 1; k >= 0; --k) {          // rows past S hold zeros
+      const float n1 = (float)(r0 + k + 1);
+      add4(s, make_float4(v[k].x / n1, v[k].y / n1, v[k].z / n1, v[k].w / n1));
+      if (r0 + k < g.S) *reinterpret_cast<float4*>(hs + (int64_t)k * g.D) = s;
+    }
+  }
+}
+
+// dc of a short sequence.  grid (nblk, B), g.brows rows each (a multiple of
+// kBlockRows): a row's dc is its running sum within its block of 8 rows plus
+// the totals of the later blocks.  Part p (see Parts) owns cr consecutive rows,
+// cr a power of two up to 8, so all in one block; it sums the totals of every
+// np-th block past the workgroup's rows, and after one barrier adds all parts'
+// sums, in part order, and the totals of the workgroup's own later blocks.
+__global__ void __launch_bounds__(kWide) mla_short_scan(const MArgs g) {
+  __shared__ float4 later[kWide];
+  const int b = (int)blockIdx.y;
+  const Parts P(g.D);
+  const int r0 = (int)blockIdx.x * g.brows;
+  const int r1 = r0 + g.brows < g.S ? r0 + g.brows : g.S;
+  int cr = 1;
+  while (cr * P.np < g.brows) cr *= 2;                   // <= 8: brows <= 64, np >= 8
+  const int c0 = r0 + P.p * cr < r1 ? r0 + P.p * cr : r1;
+  const int c1 = c0 + cr < r1 ? c0 + cr : r1;
+  const int nb = (g.S + kBlockRows - 1) / kBlockRows;    // blocks of 8 rows of the sequence
+  const int next = (r0 + g.brows) / kBlockRows;          // the first past the workgroup's rows
+  const float* __restrict__ hs = g.hs + (int64_t)b * g.S * g.D + 4 * P.col;
+  auto total = [&](int x) { return *reinterpret_cast<const float4*>(hs + (int64_t)x * kBlockRows * g.D); };
+  float4 rows[kBlockRows], near[kBlockRows];
+  float4 lat = make_float4(0.f, 0.f, 0.f, 0.f);
+  const int own = c0 / kBlockRows;                       // the block of the part's rows
+  const int nnear = (next < nb ? next : nb) - own - 1;   // later blocks of this workgroup, < 8
+  if (P.p < P.np && c0 < c1) {
+#pragma unroll
+    for (int k = 0; k < kBlockRows; ++k) {
+      if (k < cr) rows[k] = *reinterpret_cast<const float4*>(hs + (int64_t)(c0 + k < c1 ? c0 + k : c0) * g.D);
+      if (k < nnear) near[k] = total(own + 1 + k);
+    }
+  }
+  if (P.p < P.np) {
+    for (int x = next + P.p; x < nb; x += kBlockRows * P.np) {
+      float4 v[kBlockRows];
+#pragma unroll
+      for (int k = 0; k < kBlockRows; ++k) {
+        const int xx = x + k * P.np;
+        v[k] = total(xx < nb ? xx : x);
+      }
+#pragma unroll
+      for (int k = 0; k < kBlockRows; ++k)
+        if (x + k * P.np < nb) add4(lat, v[k]);
+    }
+  }
+  later[threadIdx.x] = lat;
+  __syncthreads();
+  if (P.p >= P.np || c0 >= c1) return;
+  float4 cy = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int q = 0; q < P.np; ++q) add4(cy, later[q * P.cpt + P.col]);
+#pragma unroll
+  for (int k = kBlockRows - 1; k >= 0; --k)
+    if (k < nnear) add4(cy, near[k]);
+  float* __restrict__ dcf = static_cast<float*>(g.dc) + (int64_t)b * g.S * g.ld + 4 * P.col;
+  uint16_t* __restrict__ dch = static_cast<uint16_t*>(g.dc) + (int64_t)b * g.S * g.ld + 4 * P.col;
+  const bool bf16 = g.dc_bf16 != 0;
+#pragma unroll
+  for (int k = 0; k < kBlockRows; ++k) {
+    const int r = c0 + k;
+    if (k < cr && r < c1) {
+      float4 o = cy;
+      add4(o, rows[k]);
+      if (bf16) {
+        const uint2 wv = {pack_bf16x2(o.x, o.y), pack_bf16x2(o.z, o.w)};
+        *reinterpret_cast<uint2*>(dch + (int64_t)r * g.ld) = wv;
+      } else {
+        *reinterpret_cast<float4*>(dcf + (int64_t)r * g.ld) = o;
+      }
+    }
+  }
 }
 
 bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
@@ -538,34 +679,63 @@ bool overlap(const void* a, int64_t na, const void* b, int64_t nb) {
 }
 
 constexpr int kMinK1Groups = 1024;        // K1 workgroups wanted (4 per CU)
-constexpr int64_t kCUs = 256;             // compute units of an MI355X
 constexpr int kMaxHeadSplit = 8;
 
-// Head groups for K1 when the row grid alone is small: doubles while the grid
-// has fewer than kMinK1Groups workgroups (at most 8 groups, never more than H).
-int64_t head_split(int64_t B, int64_t S, int64_t D, int64_t H) {
-  if (D < 64) return 1;
+// K1's workgroups for a column slice of D dims.
+int64_t k1_groups(int64_t B, int64_t S, int64_t D) {
   const int64_t rows_per_wg = kThreads / (D / 8);
-  const int64_t base = ((S + rows_per_wg - 1) / rows_per_wg) * B;
+  return ((S + rows_per_wg - 1) / rows_per_wg) * B;
+}
+
+// Planes of head sums the workspace is sized for.  The kernels use one; the
+// size that callers were told for a shape does not change.
+int64_t workspace_planes(int64_t B, int64_t S, int64_t D) {
+  if (D < 64) return 1;
   int64_t sp = 1;
-  while (base * sp < kMinK1Groups && sp < kMaxHeadSplit && sp * 2 <= H) sp *= 2;
+  while (k1_groups(B, S, D) * sp < kMinK1Groups && sp < kMaxHeadSplit) sp *= 2;
   return sp;
 }
 
-// Workgroups per scan block for the block totals.  Short sequences, where K1
-// splits the heads into several partial head-sum planes, leave few blocks
-// whose workgroups each read brows rows of every plane (and write the plane
-// sums back); from 128 KB per workgroup that read sets K2's length, and the
-// block is split into up to 4 column slices of at least 128 dims while K2's
-// grid (B nblk split workgroups) stays within one per CU.  Measured (B 2, H
-// 64, D 512): S 256 and 512 split 4 ways, 3-5 % faster per call; a split of
-// the single-plane S 4096 blocks (128 KB, 128 workgroups) 1 % slower.
-int32_t block_split(int64_t B, int64_t nblk, int64_t brows, int64_t hsplit, int64_t ds) {
-  if (hsplit < 2 || brows * hsplit * ds * 4 < (128 << 10)) return 1;
-  int32_t sp = 1;
-  while (sp < 4 && ds % (2 * sp * 64) == 0 && ds / (2 * sp) >= 128 && B * nblk * 2 * sp <= kCUs)
-    sp *= 2;
-  return sp;
+// Column tile of the short sequences' dO pass: the widest with at least 320
+// workgroups, whose longer contiguous pieces of a row memory serves faster;
+// else 128 dims with all of a wave's 8 or more heads in flight, unless the grid
+// with the exact rows would put two workgroups on some CUs and one on others.
+// us per call in a replayed graph, H = 64, D = 512, bf16 gradients (B x S: the tile of
+// this rule, the others in the order 512 / 256 / 128 / 64): 1 x 300, fp32 gradients:
+// 128: 17.9, others 43.4 / 29.5 / - / 25.1; 2 x 256: 64: 24.0, 43.8 / 27.9 / 27.2; 2 x
+// 512: 128: 35.3, 50.2 / 40.6 / - / 42.7; 2 x 1024: 256: 60.0, 68.5 / - / 62.4 / 69.9;
+// 2 x 1900: 512: 102.2, - / 116.6 / 111.5 / 121.9.  Before this pass (partial planes,
+// block totals, scan with the exact rows): 25.6, 28.0, 38.9, 62.1 and 109.3.
+struct ShortTile {
+  const void* kernel;
+  int cw, head_groups;
+};
+template <int CW, int U>
+ShortTile make_short_tile(bool halves) {
+  return {halves ? reinterpret_cast<const void*>(&mla_short_do<CW, U, true>)
+                 : reinterpret_cast<const void*>(&mla_short_do<CW, U, false>),
+          CW, kShortWaves * 64 / (CW / 8) / kBlockRows};
+}
+ShortTile short_tile(int64_t B, int64_t S, int64_t ds, int64_t nexact, bool halves) {
+  const int64_t blocks = B * ((S + kBlockRows - 1) / kBlockRows);
+  if (ds % 512 == 0 && blocks * (ds / 512) >= 320) return make_short_tile<512, 4>(halves);
+  if (ds % 256 == 0 && blocks * (ds / 256) >= 320) return make_short_tile<256, 4>(halves);
+  if (ds % 128 == 0 && blocks * (ds / 128) >= 320) return make_short_tile<128, 4>(halves);
+  if (ds % 128 == 0 && blocks * (ds / 128) + B * nexact <= 320) return make_short_tile<128, 8>(halves);
+  return make_short_tile<64, 4>(halves);
+}
+
+// Sequences whose K1 has fewer than kMinK1Groups workgroups are short; with
+// fp32 dq, whose stores set the pass's rate, fewer than half of that (2 x 64 x
+// 1900 x 512: K1 with U = 1, 147.9 us, against 154.1 by the short pass; 2 x 64 x
+// 1024 x 512: 84.6 against 85.0).  Where only 64-dim tiles fit, few heads leave
+// their 8 head groups one or two heads each, and many such workgroups cost more
+// than K1 (1 x 8 x 3000 x 448: 22.4 us against 30.9; 1 x 8 x 1500 x 448, 1316
+// workgroups: 18.2 against 17.8).
+bool is_short(int64_t B, int64_t H, int64_t S, int64_t ds, bool halves) {
+  if (k1_groups(B, S, ds) >= (halves ? kMinK1Groups / 2 : kMinK1Groups)) return false;
+  const int64_t blocks = B * ((S + kBlockRows - 1) / kBlockRows);
+  return ds % 128 == 0 || H >= 16 || blocks * (ds / 64) <= 1500;
 }
 
 // Rows per scan block: S / 64 rounded up to a multiple of 16, within [16, 64],
@@ -588,8 +758,7 @@ int64_t workspace_bytes(int64_t B, int64_t S, int64_t D) {
   if (B < 0 || S < 0 || D < 0 || B > (1 << 20) || S > (1ll << 31) || D > (1ll << 31)) return -1;
   const int64_t nblk = (S + block_rows(S) - 1) / block_rows(S);
   auto slice_bytes = [&](int64_t w) {
-    const int64_t sp = head_split(B, S, w, kMaxHeadSplit);   // the most any H can use
-    return (sp * B * S + B * nblk) * w * 4;
+    return (workspace_planes(B, S, w) * B * S + B * nblk) * w * 4;
   };
   const int64_t a = slice_bytes(D < kSliceD ? D : kSliceD);
   const int64_t b = D > kSliceD && D % kSliceD ? slice_bytes(D % kSliceD) : 0;
@@ -670,42 +839,47 @@ int launch(const void* q, const void* c_kv, const void* out, const void* dout, c
     g.lse = lse;
     g.dq = static_cast<uint8_t*>(dq) + col * qb;   // K1's rows; the exact rows run with col = 0
     g.dc = static_cast<uint8_t*>(dc_kv) + col * cb;
-    const int64_t hsplit = head_split(B, S, ds, H);
-    g.hps = (int32_t)((H + hsplit - 1) / hsplit);
-    g.hsplit = (int32_t)((H + g.hps - 1) / g.hps);        // non-empty head groups
     g.hs = static_cast<float*>(workspace);
-    g.hs_split = B * S * ds;
     g.brows = (int32_t)block_rows(S);
     g.nblk = (int32_t)((S + g.brows - 1) / g.brows);
-    g.tot = g.hs + g.hsplit * B * S * ds;
+    g.tot = g.hs + B * S * ds;
     g.H = (int32_t)H;
     g.S = (int32_t)S;
     g.D = (int32_t)ds;
     g.ld = (int32_t)D;
     g.nexact = sl == 0 ? (int32_t)H : 0;
-    const int32_t bsplit = block_split(B, g.nblk, g.brows, g.hsplit, ds);
-    g.bsplit_sh = bsplit == 4 ? 2 : bsplit == 2 ? 1 : 0;
     g.erows = (int32_t)(S < kE ? S : kE);
     g.scale = sm_scale;
     g.dq_bf16 = dq_dtype == FAGQ_MLA_BF16;
     g.dc_bf16 = dc_dtype == FAGQ_MLA_BF16;
     void* args[] = {&g};
-    const int rows_per_wg = kThreads / (int)(ds / 8);
-    const dim3 k1_grid((unsigned)((S + rows_per_wg - 1) / rows_per_wg), (unsigned)B,
-                       (unsigned)g.hsplit);
-    const bool k1_wide = (int64_t)k1_grid.x * k1_grid.y * k1_grid.z <= kMinK1Groups;
     const bool halves = dq_dtype == FAGQ_MLA_F32;
-    const void* k1 = halves ? (k1_wide ? reinterpret_cast<const void*>(&mla_stream_do<8, true>)
-                                       : reinterpret_cast<const void*>(&mla_stream_do<1, true>))
-                            : (k1_wide ? reinterpret_cast<const void*>(&mla_stream_do<8, false>)
-                                       : reinterpret_cast<const void*>(&mla_stream_do<2, false>));
+    const int64_t groups = k1_groups(B, S, ds);
+    if (is_short(B, H, S, ds, halves)) {
+      const ShortTile tile = short_tile(B, S, ds, g.nexact, halves);
+      const int64_t blocks = (S + kBlockRows - 1) / kBlockRows * (ds / tile.cw);
+      const size_t join = (size_t)tile.head_groups * kBlockRows * tile.cw * 4;
+      const size_t exact = g.nexact ? exact_lds_bytes(D) : 0;
+      // nexact + blocks < 2^17 + 2^26: H S D 4 < 2^32 and D >= 64.
+      int ls = launch_kernel(tile.kernel, dim3((unsigned)(g.nexact + blocks), (unsigned)B),
+                             dim3(64 * kShortWaves), args, join > exact ? join : exact, st);
+      if (ls != FAGQ_OK) return ls;
+      ls = launch_kernel(reinterpret_cast<const void*>(&mla_short_scan),
+                         dim3((unsigned)g.nblk, (unsigned)B), dim3(kWide), args, 0, st);
+      if (ls != FAGQ_OK) return ls;
+      continue;
+    }
+    const int rows_per_wg = kThreads / (int)(ds / 8);
+    const dim3 k1_grid((unsigned)((S + rows_per_wg - 1) / rows_per_wg), (unsigned)B);
+    const void* k1 = halves                    ? reinterpret_cast<const void*>(&mla_stream_do<1, true>)
+                     : groups <= kMinK1Groups ? reinterpret_cast<const void*>(&mla_stream_do<8, false>)
+                                              : reinterpret_cast<const void*>(&mla_stream_do<2, false>);
     int ls = launch_kernel(k1, k1_grid, dim3(kThreads), args, 0, st);
     if (ls != FAGQ_OK) return ls;
-    // 4 nblk < 2^22 and nexact + nblk < 2^17 + 2^20: nblk <= S / 16 + 1 and
+    // nblk < 2^20 and nexact + nblk < 2^17 + 2^20: nblk <= S / 16 + 1 and
     // H S D 4 < 2^32 with D >= 64.
     ls = launch_kernel(reinterpret_cast<const void*>(&mla_block_totals),
-                       dim3((unsigned)(g.nblk * bsplit), (unsigned)B), dim3(kWide), args,
-                       kBlockTotalLds, st);
+                       dim3((unsigned)g.nblk, (unsigned)B), dim3(kWide), args, kBlockTotalLds, st);
     if (ls != FAGQ_OK) return ls;
     ls = launch_kernel(reinterpret_cast<const void*>(&mla_exact_rows_suffix_scan),
                        dim3((unsigned)(g.nexact + g.nblk), (unsigned)B), dim3(kWide), args,
