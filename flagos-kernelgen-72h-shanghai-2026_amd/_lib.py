@@ -144,6 +144,7 @@ def load_probe(path: str | Path | None = None) -> ctypes.CDLL:
 
 
 _fast = None          # the bound _fagq_py.launch, once looked up
+_fast_mod = None      # the bound _fagq_py module (quant, gemm, dsa, mla), with it
 _fast_tried = False
 
 
@@ -151,7 +152,7 @@ def fast_launch():
     """launch() of the CPython binding (csrc/fagq_py.cpp), bound to this
     process's libfagq.so, or None when that module is not built or does not
     import (the ctypes path then serves every call; both reach fagq_launch)."""
-    global _fast, _fast_tried
+    global _fast, _fast_mod, _fast_tried
     if _fast_tried:
         return _fast
     lib = load()          # takes _lock itself (not reentrant): before the block below
@@ -161,11 +162,36 @@ def fast_launch():
                 from . import _fagq_py
                 _fagq_py.bind(ctypes.cast(lib.fagq_launch, ctypes.c_void_p).value,
                               ctypes.cast(lib.fagq_launch_typed, ctypes.c_void_p).value)
+                _fagq_py.bind_all(*[ctypes.cast(fn, ctypes.c_void_p).value for fn in
+                                    (lib.fagq_launch_parts, lib.fagq_gemm_launch,
+                                     lib.fagq_dsa_topk_launch, lib.fagq_mla_bwd_workspace_bytes,
+                                     lib.fagq_mla_bwd_launch)])
                 _fast = _fagq_py.launch
+                _fast_mod = _fagq_py
             except ImportError:
                 _fast = None
             _fast_tried = True
     return _fast
+
+
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
+def fast_module(t):
+    """(the binding's module, the current stream) for a call on tensor t, or (None,
+    None) where the Python path has to take it: without the binding, or when t is
+    not a tensor on the current GPU."""
+    if type(t) is not torch.Tensor or _raw_stream is None or _raw_device is None:
+        return None, None
+    dev = t.get_device()
+    if dev < 0 or _raw_device() != dev:
+        return None, None
+    if not _fast_tried:
+        fast_launch()
+    if _fast_mod is None:
+        return None, None
+    return _fast_mod, _raw_stream(dev)
 
 
 FAST_ARG_ERROR = 1000   # _fagq_py.ARG_ERROR: a tensor argument was rejected by the binding

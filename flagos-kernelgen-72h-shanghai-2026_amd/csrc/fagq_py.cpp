@@ -1,33 +1,43 @@
-// fagq_py.cpp - CPython binding of the operator's per-call path.
+// fagq_py.cpp - CPython binding of the operators' per-call paths.
 //
-// The Python operator (ops.fused_add_rmsnorm_group_quant, the drop-in for
-// src/task01_fused_add_rmsnorm_group_quant.py:1731-1741) spends most of a
-// decode-sized call on the host: some 30 tensor attribute reads in Python and
-// a 16-argument ctypes call cost about 5 us against a 3 us kernel.  This
-// module does the same checks on the tensors' C++ metadata and calls
-// fagq_launch (bf16 tensors) or fagq_launch_typed (fp16 activations or an
-// fp32 residual stream; include/fagq.h) through function pointers handed
-// over from the ctypes binding at import, so both bindings reach the one
-// library.
+// Small calls are bound by the host: in Python the checks (some 30 tensor
+// attribute reads), the outputs' allocation and a 16-argument ctypes call cost
+// 5 to 11 us against kernels of 3 to 8.  This module does the same checks on the
+// tensors' C++ metadata, allocates through ATen and calls the library through
+// function pointers handed over from the ctypes binding at import, so both
+// bindings reach the one library.  us per call, Python path -> this one:
+// functional quantizer 4 x 8192 8.1 -> 6.6, GEMM 32 x 4096 x 7168 11.6 -> 8.2, DSA 1 x 8 x 129 x
+// 1021 11.2 -> 5.5.
 //
 //   launch(x, residual, gamma, residual_out, norm_out, x_q, x_scale, eps,
 //          group_size, rounding, stream) -> int
+//     The drop-in for src/task01_fused_add_rmsnorm_group_quant.py:1731-1741.
 //     rounding: -1 = the format's default (fp8 RNE, int8 truncation),
 //               0 = RNE, 1 = truncation, anything else = invalid.
 //     Returns fagq_launch's status, or kArgError when a tensor argument is
 //     rejected here (the Python layer then raises its detailed error).
-//     The caller passes the current stream of the tensors' device and has
-//     made that device current.
+//   quant(...), parts(...), gemm(...), dsa(...), mla(...): the other operators,
+//     allocation included.  They return the outputs (dsa and mla: 0), the
+//     library's status as an int where it is an error, or kArgError for any
+//     argument that the Python layer should look at: it then takes the call from
+//     the start, with the same results and its own wording of the errors.
+//     Nothing is allocated or launched before all arguments are accepted.
 //
-// No device work happens here and nothing is allocated: the launch is
-// fagq_launch's.
+// In all of them the caller passes the current stream of the tensors' device
+// and has made that device current.
 #include <Python.h>
 
+#include <ATen/ATen.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "fagq.h"
+#include "fagq_dsa.h"
+#include "fagq_gemm.h"
+#include "fagq_mla.h"
 
 namespace {
 
@@ -40,6 +50,11 @@ using TypedLaunchFn = int (*)(const void*, const void*, const void*, void*, void
                               void*);
 LaunchFn g_launch = nullptr;
 TypedLaunchFn g_launch_typed = nullptr;
+decltype(&fagq_launch_parts) g_parts = nullptr;
+decltype(&fagq_gemm_launch) g_gemm = nullptr;
+decltype(&fagq_dsa_topk_launch) g_dsa = nullptr;
+decltype(&fagq_mla_bwd_workspace_bytes) g_mla_bytes = nullptr;
+decltype(&fagq_mla_bwd_launch) g_mla = nullptr;
 
 bool is_tensor(PyObject* o) { return THPVariable_Check(o); }
 
@@ -164,6 +179,298 @@ PyObject* launch(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   return PyLong_FromLong(st == FAGQ_E_FORMAT ? kArgError : st);
 }
 
+// ------------------------------------------------------------------ with allocation
+
+PyObject* arg_error() { return PyLong_FromLong(kArgError); }
+
+// Plain tensors only: a subclass may override what the Python layer calls.
+bool is_plain(PyObject* o) { return THPVariable_CheckExact(o); }
+
+// An int argument in [lo, hi].
+bool int_arg(PyObject* o, long long lo, long long hi, long long* out) {
+  if (!PyLong_CheckExact(o)) return false;
+  *out = PyLong_AsLongLong(o);
+  if (*out == -1 && PyErr_Occurred()) {
+    PyErr_Clear();
+    return false;
+  }
+  return *out >= lo && *out <= hi;
+}
+
+// A float argument: a Python float (NaN and infinities too) or int.
+bool float_arg(PyObject* o, double* out) {
+  if (!PyFloat_CheckExact(o) && !PyLong_CheckExact(o)) return false;
+  *out = PyFloat_AsDouble(o);
+  if (*out == -1.0 && PyErr_Occurred()) {
+    PyErr_Clear();
+    return false;
+  }
+  return true;
+}
+
+bool stream_arg(PyObject* o, void** out) {
+  if (!PyLong_CheckExact(o)) return false;
+  *out = PyLong_AsVoidPtr(o);
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    return false;
+  }
+  return true;
+}
+
+// Code and scale tensors of the functional forms.
+at::Tensor empty_codes(const at::Tensor& x, int64_t M, int64_t D, bool fp8) {
+  return at::empty({M, D}, at::TensorOptions(x.device()).dtype(fp8 ? at::kFloat8_e4m3fn : at::kChar));
+}
+at::Tensor empty_scale(const at::Tensor& x, int64_t M, int64_t groups, bool ue8m0, bool col_major) {
+  const auto o = at::TensorOptions(x.device()).dtype(ue8m0 ? at::kByte : at::kFloat);
+  return col_major ? at::empty_strided({M, groups}, {1, M}, o) : at::empty({M, groups}, o);
+}
+
+PyObject* three(const at::Tensor& a, const at::Tensor& b, const at::Tensor& c) {
+  PyObject* t = PyTuple_New(3);
+  if (!t) return nullptr;
+  const at::Tensor* v[3] = {&a, &b, &c};
+  for (int i = 0; i < 3; ++i) {
+    PyObject* o = THPVariable_Wrap(*v[i]);
+    if (!o) {
+      Py_DECREF(t);
+      return nullptr;
+    }
+    PyTuple_SET_ITEM(t, i, o);
+  }
+  return t;
+}
+
+// quant(x or [x, ...], residual, weight, eps, group_size, fp8, col_major, ue8m0,
+//       rounding, inplace, stream) -> (residual_out, q, scale): the functional
+// form, or with a list the multi-input form.
+PyObject* quant(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs != 11) {
+    PyErr_SetString(PyExc_TypeError, "quant() takes 11 arguments");
+    return nullptr;
+  }
+  const bool multi = PyList_CheckExact(args[0]);
+  if (!g_launch || !g_launch_typed || !g_parts) return arg_error();
+  const Py_ssize_t n = multi ? PyList_GET_SIZE(args[0]) : 1;
+  if (n < 1 || n > FAGQ_MAX_PARTS) return arg_error();
+  PyObject* xs[FAGQ_MAX_PARTS];
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    xs[i] = multi ? PyList_GET_ITEM(args[0], i) : args[0];
+    if (!is_plain(xs[i])) return arg_error();
+  }
+  long long G, fp8, col, ue, rounding, inplace;
+  void* stream;
+  if (!is_plain(args[1]) || !is_plain(args[2]) || !PyFloat_CheckExact(args[3]) ||
+      !int_arg(args[4], 1, INT32_MAX, &G) || !int_arg(args[5], 0, 1, &fp8) ||
+      !int_arg(args[6], 0, 1, &col) || !int_arg(args[7], 0, 1, &ue) ||
+      !int_arg(args[8], -1, 1, &rounding) || !int_arg(args[9], 0, 1, &inplace) ||
+      !stream_arg(args[10], &stream))
+    return arg_error();
+  const at::Tensor& x = THPVariable_Unpack(xs[0]);
+  const at::Tensor& residual = THPVariable_Unpack(args[1]);
+  const at::Tensor& weight = THPVariable_Unpack(args[2]);
+  if (x.dim() != 2 || !x.is_cuda()) return arg_error();
+  const c10::DeviceIndex dev = x.get_device();
+  const auto shape = x.sizes();
+  const int64_t M = shape[0], D = shape[1], dshape[1] = {D};
+  const at::ScalarType at_ = x.scalar_type(), rt = residual.scalar_type();
+  const int act = dtype_code(at_), res = dtype_code(rt);
+  if (act < 0 || res < 0 || D % G != 0) return arg_error();
+  if (multi && (act != FAGQ_DT_BF16 || res != FAGQ_DT_BF16)) return arg_error();
+  for (Py_ssize_t i = 0; i < n; ++i)
+    if (!rows_ok(THPVariable_Unpack(xs[i]), shape, dev, at_)) return arg_error();
+  if (!rows_ok(residual, shape, dev, rt) ||
+      !rows_ok(weight, at::IntArrayRef(dshape, 1), dev, at_))
+    return arg_error();
+  if (fp8 && rounding == 1) return arg_error();
+  const int qf = fp8 ? FAGQ_Q_FP8_E4M3FN : FAGQ_Q_INT8;
+  const int rnd = fp8 || rounding == 0 ? FAGQ_ROUND_RNE : FAGQ_ROUND_TRUNC;
+  const int sf = ue ? FAGQ_SCALE_UE8M0 : FAGQ_SCALE_F32;
+  const int64_t groups = D / G;
+
+  const at::Tensor residual_out = inplace ? residual : at::empty_like(residual);
+  const at::Tensor q = empty_codes(x, M, D, fp8);
+  const at::Tensor scale = empty_scale(x, M, groups, ue, col);
+  if (M != 0) {
+    // A [M, groups] tensor with one row or column is both: row-major, as in Python.
+    const int layout = scale.is_contiguous() ? FAGQ_LAYOUT_ROW_MAJOR : FAGQ_LAYOUT_COL_MAJOR;
+    const float eps = (float)PyFloat_AS_DOUBLE(args[3]);
+    int st;
+    if (multi) {
+      const void* ptrs[FAGQ_MAX_PARTS];
+      for (Py_ssize_t i = 0; i < n; ++i) ptrs[i] = THPVariable_Unpack(xs[i]).data_ptr();
+      st = g_parts(ptrs, (int)n, residual.data_ptr(), weight.data_ptr(), residual_out.data_ptr(),
+                   q.data_ptr(), scale.data_ptr(), M, D, G, eps, qf, sf, layout, rnd, stream);
+    } else if (act == FAGQ_DT_BF16 && res == FAGQ_DT_BF16) {
+      st = g_launch(x.data_ptr(), residual.data_ptr(), weight.data_ptr(), residual_out.data_ptr(),
+                    nullptr, q.data_ptr(), scale.data_ptr(), M, D, G, eps, qf, sf, layout, rnd,
+                    stream);
+    } else {
+      st = g_launch_typed(x.data_ptr(), residual.data_ptr(), weight.data_ptr(),
+                          residual_out.data_ptr(), nullptr, q.data_ptr(), scale.data_ptr(), M, D,
+                          G, eps, qf, sf, layout, rnd, act, res, stream);
+      if (st == FAGQ_E_FORMAT) return arg_error();       // a type pair the library refuses
+    }
+    if (st != FAGQ_OK) return PyLong_FromLong(st);
+  }
+  return three(residual_out, q, scale);   // inplace: the caller's own tensor object
+  END_HANDLE_TH_ERRORS
+}
+
+// gemm(a_q, a_scale, b_q, b_scale, out or None, stream) -> out
+PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs != 6) {
+    PyErr_SetString(PyExc_TypeError, "gemm() takes 6 arguments");
+    return nullptr;
+  }
+  if (!g_gemm) return arg_error();
+  for (int i = 0; i < 4; ++i)
+    if (!is_plain(args[i])) return arg_error();
+  const bool has_out = args[4] != Py_None;
+  void* stream;
+  if ((has_out && !is_plain(args[4])) || !stream_arg(args[5], &stream)) return arg_error();
+  const at::Tensor& a = THPVariable_Unpack(args[0]);
+  const at::Tensor& as = THPVariable_Unpack(args[1]);
+  const at::Tensor& b = THPVariable_Unpack(args[2]);
+  const at::Tensor& bs = THPVariable_Unpack(args[3]);
+  if (a.dim() != 2 || b.dim() != 2 || !a.is_cuda()) return arg_error();
+  const c10::DeviceIndex dev = a.get_device();
+  const int64_t M = a.size(0), K = a.size(1), N = b.size(0), kb = K / 128, nb = (N + 127) / 128;
+  if (b.size(1) != K || K % 128 != 0 || N % 16 != 0) return arg_error();
+  const int64_t ashape[2] = {M, K}, bshape[2] = {N, K}, sshape[2] = {nb, kb}, cshape[2] = {M, N};
+  auto scale_format = [](const at::Tensor& t) {
+    return t.scalar_type() == at::kFloat  ? FAGQ_SCALE_F32
+           : t.scalar_type() == at::kByte ? FAGQ_SCALE_UE8M0
+                                          : -1;
+  };
+  const int asf = scale_format(as), bsf = scale_format(bs);
+  if (asf < 0 || bsf < 0 || !rows_ok(a, ashape, dev, at::kFloat8_e4m3fn) ||
+      !rows_ok(b, bshape, dev, at::kFloat8_e4m3fn) || !rows_ok(bs, sshape, dev, bs.scalar_type()) ||
+      as.dim() != 2 || as.size(0) != M || as.size(1) != kb || !as.is_cuda() ||
+      as.get_device() != dev)
+    return arg_error();
+  int layout;
+  if (as.is_contiguous()) layout = FAGQ_LAYOUT_ROW_MAJOR;
+  else if (as.stride(0) == 1 && as.stride(1) == M) layout = FAGQ_LAYOUT_COL_MAJOR;
+  else return arg_error();
+  if (has_out && !rows_ok(THPVariable_Unpack(args[4]), cshape, dev, at::kBFloat16)) return arg_error();
+  const at::Tensor out = has_out ? THPVariable_Unpack(args[4])
+                                 : at::empty({M, N}, at::TensorOptions(a.device()).dtype(at::kBFloat16));
+  const int st = g_gemm(a.data_ptr(), as.data_ptr(), b.data_ptr(), bs.data_ptr(), out.data_ptr(), M,
+                        N, K, asf, layout, bsf, stream);
+  if (st != FAGQ_OK) return PyLong_FromLong(st);
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
+// dsa(scores, page_table, q_pos, kv_lens, out_blocks, out_pages, block_size,
+//     top_k, stream) -> status
+PyObject* dsa(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs != 9) {
+    PyErr_SetString(PyExc_TypeError, "dsa() takes 9 arguments");
+    return nullptr;
+  }
+  if (!g_dsa) return arg_error();
+  for (int i = 0; i < 6; ++i)
+    if (!is_plain(args[i])) return arg_error();
+  long long bs, k;
+  void* stream;
+  if (!int_arg(args[6], INT64_MIN, INT64_MAX, &bs) || !int_arg(args[7], INT64_MIN, INT64_MAX, &k) ||
+      !stream_arg(args[8], &stream))
+    return arg_error();
+  const at::Tensor& s = THPVariable_Unpack(args[0]);
+  if (s.dim() != 4 || !s.is_cuda() || !s.is_contiguous()) return arg_error();
+  const c10::DeviceIndex dev = s.get_device();
+  const int64_t B = s.size(0), H = s.size(1), Q = s.size(2), NB = s.size(3);
+  const int sdt = s.scalar_type() == at::kFloat      ? FAGQ_DSA_F32
+                  : s.scalar_type() == at::kBFloat16 ? FAGQ_DSA_BF16
+                                                     : -1;
+  const at::Tensor* t[5];
+  for (int i = 0; i < 5; ++i) t[i] = &THPVariable_Unpack(args[1 + i]);
+  const at::ScalarType it = t[1]->scalar_type();
+  if (sdt < 0 || (it != at::kInt && it != at::kLong)) return arg_error();
+  const int64_t pt[2] = {B, NB}, qp[2] = {B, Q}, kv[1] = {B}, ob[4] = {B, H, Q, k};
+  if (!rows_ok(*t[0], pt, dev, at::kInt) || !rows_ok(*t[1], qp, dev, it) ||
+      !rows_ok(*t[2], at::IntArrayRef(kv, 1), dev, it) || !rows_ok(*t[3], ob, dev, at::kInt) ||
+      !rows_ok(*t[4], ob, dev, at::kInt))
+    return arg_error();
+  return PyLong_FromLong(g_dsa(s.data_ptr(), sdt, t[0]->data_ptr(), t[1]->data_ptr(),
+                               t[2]->data_ptr(), it == at::kLong ? FAGQ_DSA_I64 : FAGQ_DSA_I32,
+                               t[3]->data_ptr(), t[4]->data_ptr(), B, H, Q, NB, bs, k, stream));
+  END_HANDLE_TH_ERRORS
+}
+
+// mla(q, c_kv, out, do, lse, dq, dc_kv, sm_scale, stream) -> status; the
+// workspace is allocated here (a caller's own goes through Python).
+PyObject* mla(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs != 9) {
+    PyErr_SetString(PyExc_TypeError, "mla() takes 9 arguments");
+    return nullptr;
+  }
+  if (!g_mla || !g_mla_bytes) return arg_error();
+  for (int i = 0; i < 7; ++i)
+    if (!is_plain(args[i])) return arg_error();
+  double sm_scale;
+  void* stream;
+  if (!float_arg(args[7], &sm_scale) || !stream_arg(args[8], &stream)) return arg_error();
+  const at::Tensor* t[7];
+  for (int i = 0; i < 7; ++i) t[i] = &THPVariable_Unpack(args[i]);
+  if (t[0]->dim() != 4 || !t[0]->is_cuda()) return arg_error();
+  const c10::DeviceIndex dev = t[0]->get_device();
+  const auto qs = t[0]->sizes();
+  const int64_t B = qs[0], H = qs[1], S = qs[2], D = qs[3];
+  const int64_t cs[3] = {B, S, D}, ls[3] = {B, H, S};
+  auto grad_code = [](const at::Tensor& g) {
+    return g.scalar_type() == at::kFloat      ? FAGQ_MLA_F32
+           : g.scalar_type() == at::kBFloat16 ? FAGQ_MLA_BF16
+                                              : -1;
+  };
+  const int dq = grad_code(*t[5]), dc = grad_code(*t[6]);
+  if (dq < 0 || dc < 0 || !rows_ok(*t[0], qs, dev, at::kBFloat16) ||
+      !rows_ok(*t[1], cs, dev, at::kBFloat16) || !rows_ok(*t[2], qs, dev, at::kBFloat16) ||
+      !rows_ok(*t[3], qs, dev, at::kBFloat16) || !rows_ok(*t[4], ls, dev, at::kFloat) ||
+      !rows_ok(*t[5], qs, dev, t[5]->scalar_type()) || !rows_ok(*t[6], cs, dev, t[6]->scalar_type()))
+    return arg_error();
+  const int64_t need = g_mla_bytes(B, S, D);
+  if (need < 0) return arg_error();
+  const at::Tensor ws = at::empty({std::max<int64_t>(need, 16)},
+                                  at::TensorOptions(t[0]->device()).dtype(at::kByte));
+  return PyLong_FromLong(g_mla(t[0]->data_ptr(), t[1]->data_ptr(), t[2]->data_ptr(),
+                               t[3]->data_ptr(), static_cast<const float*>(t[4]->data_ptr()),
+                               t[5]->data_ptr(), t[6]->data_ptr(), ws.data_ptr(), ws.numel(), B, H,
+                               S, D, (float)sm_scale, dq, dc, stream));
+  END_HANDLE_TH_ERRORS
+}
+
+// bind_all(addresses of fagq_launch_parts, fagq_gemm_launch,
+// fagq_dsa_topk_launch, fagq_mla_bwd_workspace_bytes, fagq_mla_bwd_launch).
+PyObject* bind_all(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 5) {
+    PyErr_SetString(PyExc_TypeError, "bind_all() takes 5 arguments");
+    return nullptr;
+  }
+  void* p[5];
+  for (int i = 0; i < 5; ++i) {
+    p[i] = PyLong_AsVoidPtr(args[i]);
+    if (PyErr_Occurred()) return nullptr;
+    if (!p[i]) {
+      PyErr_SetString(PyExc_ValueError, "bind_all(): null function address");
+      return nullptr;
+    }
+  }
+  g_parts = reinterpret_cast<decltype(g_parts)>(p[0]);
+  g_gemm = reinterpret_cast<decltype(g_gemm)>(p[1]);
+  g_dsa = reinterpret_cast<decltype(g_dsa)>(p[2]);
+  g_mla_bytes = reinterpret_cast<decltype(g_mla_bytes)>(p[3]);
+  g_mla = reinterpret_cast<decltype(g_mla)>(p[4]);
+  Py_RETURN_NONE;
+}
+
 // bind(address of fagq_launch, address of fagq_launch_typed) in the loaded
 // libfagq.so.
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
@@ -188,9 +495,19 @@ PyMethodDef kMethods[] = {
      METH_FASTCALL, "Checks the operator's tensors and calls fagq_launch; returns its status."},
     {"bind", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&bind)),
      METH_FASTCALL, "Sets the addresses of fagq_launch and fagq_launch_typed."},
+    {"quant", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&quant)),
+     METH_FASTCALL, "The functional and multi-input quantizer: allocates and launches."},
+    {"gemm", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&gemm)),
+     METH_FASTCALL, "The fp8 block-scaled GEMM: allocates (without an out) and launches."},
+    {"dsa", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&dsa)),
+     METH_FASTCALL, "The DSA top-k page-table transform; returns its status."},
+    {"mla", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&mla)),
+     METH_FASTCALL, "The MLA backward with a workspace of its own; returns its status."},
+    {"bind_all", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&bind_all)),
+     METH_FASTCALL, "Sets the addresses of the other entry points."},
     {nullptr, nullptr, 0, nullptr}};
 
-PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_fagq_py", "Per-call binding of fagq_launch.", -1,
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_fagq_py", "Per-call binding of the operators.", -1,
                        kMethods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

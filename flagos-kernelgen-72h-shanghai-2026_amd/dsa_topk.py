@@ -30,6 +30,15 @@ def dsa_topk_page_table_transform(scores: torch.Tensor, page_table: torch.Tensor
     """scores: float32 or bfloat16 [B, H, Q, NB] contiguous; page_table: int32 [B, NB];
     q_pos: [B, Q] and kv_lens: [B], both int32 or both int64; out_blocks, out_pages:
     int32 [B, H, Q, top_k].  Returns ``(out_blocks, out_pages)``."""
+    mod, stream = _lib.fast_module(scores)
+    if mod is not None:
+        st = mod.dsa(scores, page_table, q_pos, kv_lens, out_blocks, out_pages, block_size, top_k,
+                     stream)
+        if st == 0:
+            return out_blocks, out_pages
+        if st != _lib.FAST_ARG_ERROR:
+            _lib.check(st, "fagq_dsa_topk_launch")
+        # An argument the binding leaves to the checks below.
     if scores.dim() != 4:
         raise ValueError(f"scores must be [B, H, Q, NB], got shape {tuple(scores.shape)}")
     B, H, Q, NB = (int(s) for s in scores.shape)

@@ -40,6 +40,14 @@ def fp8_block_scaled_gemm(a_q: torch.Tensor, a_scale: torch.Tensor, b_q: torch.T
     column-major (strides (1, M), as the quantizer writes it); b_q: float8_e4m3fn
     [N, K]; b_scale: float32 / uint8 [ceil(N/128), K/128] contiguous.  Returns
     (or fills) a bf16 [M, N] tensor, asynchronously on the current stream."""
+    mod, stream = _lib.fast_module(a_q)
+    if mod is not None:
+        r = mod.gemm(a_q, a_scale, b_q, b_scale, out, stream)
+        if type(r) is not int:
+            return r
+        if r != _lib.FAST_ARG_ERROR:
+            _lib.check(r, "fagq_gemm_launch")
+        # An argument the binding leaves to the checks below.
     if a_q.dtype != _FP8 or b_q.dtype != _FP8:
         raise TypeError("a_q and b_q must be float8_e4m3fn")
     if a_q.dim() != 2 or b_q.dim() != 2 or a_q.shape[1] != b_q.shape[1]:

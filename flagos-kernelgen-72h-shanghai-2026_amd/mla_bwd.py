@@ -60,6 +60,14 @@ def mla_bwd_nope_dkdv(q: torch.Tensor, c_kv: torch.Tensor, out: torch.Tensor, do
     contiguous, on one GPU.  ``workspace`` (optional): a uint8 GPU tensor of at
     least ``workspace_bytes(B, S, D)`` bytes; allocated per call when absent,
     as the reference allocates its head-sum buffer.  Returns ``(dq, dc_kv)``."""
+    mod, fast_stream = _lib.fast_module(q) if workspace is None else (None, None)
+    if mod is not None:
+        st = mod.mla(q, c_kv, out, do, lse, dq, dc_kv, sm_scale, fast_stream)
+        if st == 0:
+            return dq, dc_kv
+        if st != _lib.FAST_ARG_ERROR:
+            _lib.check(st, "fagq_mla_bwd_launch")
+        # An argument the binding leaves to the checks below.
     if q.dim() != 4:
         raise ValueError(f"q must be [B, H, S, D], got shape {tuple(q.shape)}")
     B, H, S, D = (int(s) for s in q.shape)

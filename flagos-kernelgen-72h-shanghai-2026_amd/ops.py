@@ -265,6 +265,28 @@ def empty_scales(M: int, groups: int, *, ue8m0: bool = False, col_major: bool = 
     return torch.empty(M, groups, dtype=dt, device=device)
 
 
+def _fast_quant(x, xs, residual, weight, eps, group_size, out_dtype, col_major, ue8m0, rounding,
+                inplace, what="fagq_launch"):
+    """The functional forms through the CPython binding (xs: x, or the list of partial
+    tensors): (residual_out, q, scale), or None where the Python path has to take the
+    call (see _lib.fast_module) or to word its error."""
+    mod, stream = _lib.fast_module(x)
+    if mod is None or not isinstance(rounding, (str, type(None))):
+        return None
+    fp8 = out_dtype is _FP8
+    if not fp8 and out_dtype is not _INT8:
+        return None
+    # fp8 codes are always rounded to nearest even, whatever `rounding` says.
+    r = mod.quant(xs, residual, weight, eps, group_size, 1 if fp8 else 0, 1 if col_major else 0,
+                  1 if ue8m0 else 0, 0 if fp8 else _ROUNDING_CODE.get(rounding, -2),
+                  1 if inplace else 0, stream)
+    if type(r) is tuple:
+        return r
+    if r != _lib.FAST_ARG_ERROR:
+        _lib.check(r, what)
+    return None
+
+
 def fused_add_rmsnorm_group_quant_fn(
     x: torch.Tensor,
     residual: torch.Tensor,
@@ -286,6 +308,10 @@ def fused_add_rmsnorm_group_quant_fn(
     UE8M0 bytes when ``scale_ue8m0``.  int8 codes default to round-half-even
     here (the reference-signature function defaults to truncation).
     """
+    r = _fast_quant(x, x, residual, weight, eps, group_size, out_dtype, scale_col_major,
+                    scale_ue8m0, rounding, inplace_residual)
+    if r is not None:
+        return r
     M, D = (int(s) for s in x.shape)
     residual_out = residual if inplace_residual else torch.empty_like(residual)
     q = torch.empty((M, D), dtype=out_dtype, device=x.device)
@@ -322,6 +348,10 @@ def fused_reduce_add_rmsnorm_group_quant(
     if not 1 <= len(parts) <= 8:
         raise ValueError(f"x_parts must hold 1 to 8 tensors, got {len(parts)}")
     x0 = parts[0]
+    r = _fast_quant(x0, parts, residual, weight, eps, group_size, out_dtype, scale_col_major,
+                    scale_ue8m0, rounding, inplace_residual, "fagq_launch_parts")
+    if r is not None:
+        return r
     if x0.dim() != 2:
         raise ValueError(f"x_parts[0] must be 2-D [M, D], got shape {tuple(x0.shape)}")
     if not x0.is_cuda:
