@@ -129,6 +129,18 @@ __device__ __forceinline__ uint32_t wave_reduce(uint32_t v, Op op) {
   }
   return v;
 }
+// The same over each N consecutive lanes (4 or 16).
+template <int N, class Op>
+__device__ __forceinline__ uint32_t reduce_slots(uint32_t v, Op op) {
+  static_assert(N == 4 || N == 16, "quads or 16-lane rows");
+  v = op(v, dpp<0xB1>(v));
+  v = op(v, dpp<0x4E>(v));
+  if constexpr (N == 16) {
+    v = op(v, dpp<0x141>(v));
+    v = op(v, dpp<0x140>(v));
+  }
+  return v;
+}
 struct UMax {
   __device__ uint32_t operator()(uint32_t a, uint32_t b) const { return a > b ? a : b; }
 };
@@ -370,6 +382,7 @@ __global__ void __launch_bounds__(KIND == kSmallRows ? 64 * kSmallWaves : 64 * k
 dsa_topk_rows(const DArgs g) {
   constexpr bool MULTI = KIND == kLongRows;
   constexpr int VEC = BF16 ? 8 : 4;
+  constexpr int kSlots = KIND == kSmallRows ? kSmallWaves : kMaxWaves;   // waves of a workgroup
   __shared__ Lds<CAP> lds;
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -460,9 +473,15 @@ dsa_topk_rows(const DArgs g) {
     lds.kslot[w][1] = kmin;
   }
   __syncthreads();
-  for (int x = 0; x < nwv; ++x) {
-    kmax = kmax > lds.kslot[x][0] ? kmax : lds.kslot[x][0];
-    kmin = kmin < lds.kslot[x][1] ? kmin : lds.kslot[x][1];
+  // Lane x takes wave x's partials; the reduction then spans the live waves'
+  // lanes.  A loop over the waves was one LDS round trip each on the row's
+  // serial chain: 75.5 -> 73.6 us at 2 x 32 x 512 rows of 4096 (4 waves) and
+  // 8.85 -> 8.48 us at 256 rows of 16384 (16 waves).
+  {
+    const int x = lane & (kSlots - 1);
+    const uint2 k = *reinterpret_cast<const uint2*>(lds.kslot[x]);
+    kmax = reduce_slots<kSlots>(x < nwv ? k.x : 0u, UMax());
+    kmin = reduce_slots<kSlots>(x < nwv ? k.y : ~0u, UMin());
   }
   vmax = ord_val(kmax);
   vmin = ord_val(kmin);
@@ -671,6 +690,12 @@ dsa_topk_rows(const DArgs g) {
     __syncthreads();
   }
 
+  // Only score loads that no one reads can still be in flight here (chunks past
+  // the row's end): a wait that costs nothing.  Without it the compiler puts one
+  // at the head of the rank loop, where it also waits for the stores of the pass
+  // before.  top_k 512 and 1024 of 4096 (2 x 32 x 512 rows) take several passes:
+  // 127.4 -> 122.0 us and 188.7 -> 178.2 us.
+  __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0), the other counters untouched
   // Ranks: each candidate counts the candidates of its segment ahead of it.
   const int64_t ob = row * K;
   for (uint32_t i = (uint32_t)t; i < nc; i += (uint32_t)stride) {
