@@ -185,25 +185,28 @@ __device__ __forceinline__ float scale_value(uint32_t s) {
   return SF == SF_UE8M0 ? e8m0_to_f32(s) : __uint_as_float(s);
 }
 
-// One k-block's products of TN x TM tiles: weight fragments bf with scale sb,
-// activation fragments af with the lane's row scales sa.  Both UE8M0: the
+// One k-block's products of TN x TM tiles: weight fragments bf with scale sb[0],
+// or each its own of TN, activation fragments af with the lane's row scales sa.  Both UE8M0: the
 // matrix core applies the scales; else each product goes to a temporary and is
 // added as fmaf(t, sa * sb, acc).
-template <int ASF, int BSF, int TM, int TN>
+template <int ASF, int BSF, int TM, int TN, int NB>
 __device__ __forceinline__ void products(f32x4 (&acc)[TN][TM], const i32x8 (&bf)[TN],
-                                         const i32x8 (&af)[TM], uint32_t sb,
+                                         const i32x8 (&af)[TM], const uint32_t (&sb)[NB],
                                          const uint32_t (&sa)[TM]) {
+  static_assert(NB == 1 || NB == TN, "one weight scale or one per tile");
   if constexpr (ASF == SF_UE8M0 && BSF == SF_UE8M0) {
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int t = 0; t < TM; ++t)
         acc[j][t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-            bf[j], af[t], acc[j][t], 0, 0, 0, (int)sb, 0, (int)sa[t]);
+            bf[j], af[t], acc[j][t], 0, 0, 0, (int)sb[NB == 1 ? 0 : j], 0, (int)sa[t]);
   } else {
-    float sm[TM];
+    float sm[NB][TM];
 #pragma unroll
-    for (int t = 0; t < TM; ++t) sm[t] = scale_value<ASF>(sa[t]) * scale_value<BSF>(sb);
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int t = 0; t < TM; ++t) sm[i][t] = scale_value<ASF>(sa[t]) * scale_value<BSF>(sb[i]);
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
@@ -211,7 +214,7 @@ __device__ __forceinline__ void products(f32x4 (&acc)[TN][TM], const i32x8 (&bf)
         const f32x4 p = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
             bf[j], af[t], f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0, 127, 0, 127);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[j][t][e] = __builtin_fmaf(p[e], sm[t], acc[j][t][e]);
+        for (int e = 0; e < 4; ++e) acc[j][t][e] = __builtin_fmaf(p[e], sm[NB == 1 ? 0 : j][t], acc[j][t][e]);
       }
   }
 #pragma unroll
@@ -549,9 +552,11 @@ int pick_bn(int64_t M, int64_t N) {
 // 256 .. 4096, K 512 .. 7168 with fp32 and UE8M0 scales (MI355X, 384 shapes, replayed graphs,
 // operands rotated): 80 % of the points within 15 %, and the choice by these
 // numbers took 0.6 % longer than the fastest tile of each shape (geometric mean),
-// 11 % at worst.
+// 11 % at worst.  96 x 96 came after these: 140 further points, M 500 .. 4096; of
+// the 20 it is chosen at, each is faster than with the others: 1000 x 2112, where
+// 128 x 128 leaves 120 CUs idle, 17 .. 20 % (K 512 .. 7168), 2000 x 2112 5 .. 15 %.
 enum SmallTile { kWaves16x16, kWaves32x32, kWaves32x64, kRing64x64, kRing128x64, kRing128x128,
-                 kRing192x128, kNumSmall, kNoSmall = -1 };
+                 kRing192x128, kRing96x96, kNumSmall, kNoSmall = -1 };
 struct SmallInfo {
   int bm, bn, threads;
   double c0, t0, c1, t1;
@@ -560,11 +565,12 @@ constexpr SmallInfo kSmall[kNumSmall] = {
     {16, 16, 512, 2.76, 0.043, 0.27, 0.045},  {32, 32, 512, 2.97, 0.078, 0.60, 0.098},
     {32, 64, 512, 3.46, 0.124, 2.04, 0.150},  {64, 64, 256, 3.26, 0.233, 1.36, 0.170},
     {128, 64, 512, 3.63, 0.334, 2.02, 0.281}, {128, 128, 512, 4.73, 0.490, 4.03, 0.569},
-    {192, 128, 512, 6.35, 0.673, 6.12, 0.779}};
+    {192, 128, 512, 6.35, 0.673, 6.12, 0.779}, {96, 96, 256, 4.12, 0.389, 2.16, 0.254}};
 using Ring64x64 = Ring<2, 2, 2, 2, 5>;       // two workgroups per CU
 using Ring128x64 = Ring<2, 2, 4, 2, 3>;      // two workgroups per CU
 using Ring128x128 = Ring<2, 4, 4, 2, 3>;
 using Ring192x128 = Ring<3, 4, 4, 2, 4>;
+using Ring96x96 = Ring<3, 3, 2, 2, 3>;       // two workgroups per CU
 // The same for one round of 256-row tiles, 256 and 192 columns wide.
 constexpr double kPP256C = 13.0, kPP256T = 1.368, kPP192C = 6.87, kPP192T = 0.923;
 constexpr int64_t kSmallMinBlocks = 4;       // k-blocks: the fits' range ends at K = 512
@@ -609,8 +615,10 @@ const void* small_kernel(int tile) {
       return reinterpret_cast<const void*>(&fagq_gemm_ring_kernel<ASF, BSF, Ring128x64>);
     case kRing128x128:
       return reinterpret_cast<const void*>(&fagq_gemm_ring_kernel<ASF, BSF, Ring128x128>);
-    default:
+    case kRing192x128:
       return reinterpret_cast<const void*>(&fagq_gemm_ring_kernel<ASF, BSF, Ring192x128>);
+    default:
+      return reinterpret_cast<const void*>(&fagq_gemm_ring_kernel<ASF, BSF, Ring96x96>);
   }
 }
 const void* small_kernel_for(int tile, int asf, int bsf) {

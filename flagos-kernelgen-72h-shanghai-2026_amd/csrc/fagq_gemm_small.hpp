@@ -11,8 +11,9 @@
 //   fagq_gemm_ring_kernel - the waves split the tile, and share a ring of
 //     k-blocks in LDS.  For the larger tiles, whose accumulators one wave cannot
 //     hold.
-// No tile is wider than 128 columns nor starts off a multiple of its width, so
-// a tile's columns lie in one 128-column weight block.
+// No tile is wider than 128 columns.  The columns of those whose width divides
+// 128 lie in one 128-column weight block; a 96-column tile may straddle two, and
+// each of its 16-column tiles takes its own block's scale.
 
 // ------------------------------------------------------------------ K split over waves
 
@@ -115,7 +116,8 @@ __global__ void __launch_bounds__(64 * W) fagq_gemm_waves_kernel(const GArgs g) 
 #pragma unroll
     for (int t = 0; t < TM; ++t) af[t] = lds_frag(stage, 16 * (TN + t) + r, lane);
     issue_order_fence();
-    products<ASF, BSF>(acc, bf, af, sb, sa);
+    const uint32_t sbs[1] = {sb};
+    products<ASF, BSF>(acc, bf, af, sbs, sa);
   };
 
   Block x[U];
@@ -171,7 +173,9 @@ __global__ void __launch_bounds__(64 * W) fagq_gemm_waves_kernel(const GArgs g) 
 // (WM + 1) 16 TN WN cycles a k-block against MFMA's 8 TM TN WM WN.  us per call,
 // UE8M0, 256-row tiles before and this kernel: 256 x 4096 x 7168 55.4 -> 16.0
 // (64 x 64), 512 x 4096 x 7168 55.7 -> 23.0 (128 x 64), 1000 x 2112 x 7168 56.4
-// -> 30.2 (128 x 128), 1500 x 4096 x 7168 57.3 -> 46.4 (192 x 128).
+// -> 25.5 (96 x 96; 128 x 128: 30.2), 1500 x 4096 x 7168 57.3 -> 46.4 (192 x 128).
+// The 96 x 96 tile with 6 waves: 24.8 .. 27.7 there, but 46 against 41 us at 2048 x 2112 x
+// 7168, where two workgroups share a CU; 4 waves with 4 or 6 stages 29.5 and 32.0.
 template <int TM_, int TN_, int WM_, int WN_, int S_>
 struct Ring {
   static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, S = S_;
@@ -179,8 +183,9 @@ struct Ring {
   static constexpr int STAGE = (BM + BN) * kBK;
   static constexpr int PER_CU = 160 * 1024 / (S * STAGE);          // workgroups by LDS
   static constexpr int COPIES = (BM + BN) / 8 / WAVES;             // 1 KB copies per wave and stage
+  static constexpr int NB = 128 % BN ? 2 : 1;                      // weight blocks of a wave's columns
   static_assert(COPIES * WAVES * 8 == BM + BN, "the waves share a stage's copies evenly");
-  static_assert(S >= 3 && PER_CU >= 1 && 128 % BN == 0 && (S - 1) * (COPIES + TM + 1) < 64,
+  static_assert(S >= 3 && PER_CU >= 1 && BN <= 128 && (S - 1) * (COPIES + TM + NB) < 64,
                 "ring geometry");
 };
 
@@ -188,7 +193,7 @@ template <int ASF, int BSF, class R>
 __global__ void __launch_bounds__(64 * R::WAVES, R::PER_CU * R::WAVES / 4)
 fagq_gemm_ring_kernel(const GArgs g) {
   constexpr int TM = R::TM, TN = R::TN, S = R::S, C = R::COPIES;
-  constexpr int kScaleLoads = TM + 1;                    // memory instructions of load_scales
+  constexpr int kScaleLoads = TM + R::NB;                    // memory instructions of load_scales
   __shared__ __attribute__((aligned(1024))) uint8_t lds[S * R::STAGE];
 
   const int lane = threadIdx.x & 63;
@@ -229,14 +234,19 @@ fagq_gemm_ring_kernel(const GArgs g) {
   const int r = lane & 15;
   const uint32_t as_voff = (uint32_t)(m0 + wm * 16 * TM + r) * (uint32_t)g.as_mstride * asb;
   const int wcol = n0 + wn * 16 * TN;
+  // The wave's column tiles from jsplit on lie in the next weight block (NB 2).
+  // Past the last column that may be no block of B at all: out of range, zero.
   const uint32_t bs_row = (uint32_t)(wcol >> 7) * (uint32_t)g.kblocks;
+  const int jsplit = ((wcol & -128) + 128 - wcol) / 16;
   struct Scales {
-    uint32_t b, a[TM];
+    uint32_t b[R::NB], a[TM];
   };
   auto load_scales = [&](int kb) {
     const int kc = kb < last ? kb : last;
     Scales s;
-    s.b = load_scale<BSF>(rbs, (bs_row + (uint32_t)kc) * bsb);
+#pragma unroll
+    for (int i = 0; i < R::NB; ++i)
+      s.b[i] = load_scale<BSF>(rbs, (bs_row + (uint32_t)(i * g.kblocks + kc)) * bsb);
 #pragma unroll
     for (int t = 0; t < TM; ++t)
       s.a[t] = load_scale<ASF>(ras, as_voff + ((uint32_t)kc * (uint32_t)g.as_kstride +
@@ -285,7 +295,11 @@ fagq_gemm_ring_kernel(const GArgs g) {
     issue_order_fence();
     read_frags((p + 1) % S, bf[(p + 1) % 2], af[(p + 1) % 2]);
     __builtin_amdgcn_sched_barrier(0);
-    products<ASF, BSF>(acc, bf[p % 2], af[p % 2], s.b, s.a);
+    constexpr int kB = R::NB == 1 ? 1 : TN;
+    uint32_t sb[kB];
+#pragma unroll
+    for (int j = 0; j < kB; ++j) sb[j] = R::NB == 1 || j < jsplit ? s.b[0] : s.b[R::NB - 1];
+    products<ASF, BSF>(acc, bf[p % 2], af[p % 2], sb, s.a);
     __builtin_amdgcn_sched_barrier(0);
   };
   bool more = true;                                      // uniform over the workgroup

@@ -44,10 +44,11 @@ FAGQ_API int fagq_launch_mapped(const void* x, const void* residual, const void*
 /* fagq_gemm_launch with the tile width forced: block_n 192 or 256 columns
  * of C per workgroup of 256 rows (0: the shape's own choice, as
  * fagq_gemm_launch).  Both widths give the same bits: each output takes the
- * same MFMA and scale sequence.  block_n = 1 .. 7 forces one of the tiles for
+ * same MFMA and scale sequence.  block_n = 1 .. 8 forces one of the tiles for
  * small products instead (16 x 16, 32 x 32, 32 x 64, then 64 x 64, 128 x 64, 128 x
- * 128 and 192 x 128, which give the 256-row tiles' bits; M, N and K at most 65536,
- * else FAGQ_E_TOO_LARGE).  Other arguments and rules as fagq_gemm_launch (fagq_gemm.h);
+ * 128, 192 x 128 and 96 x 96, which give the 256-row tiles' bits; M, N and K at most
+ * 65536, else FAGQ_E_TOO_LARGE).  Other arguments and rules as fagq_gemm_launch
+ * (fagq_gemm.h);
  * FAGQ_E_FORMAT for another block_n. */
 FAGQ_API int fagq_gemm_launch_mapped(const void* a_q, const void* a_scale, const void* b_q,
                                      const void* b_scale, void* c, int64_t M, int64_t N,

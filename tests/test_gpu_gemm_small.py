@@ -16,7 +16,7 @@ from tests.test_gpu_gemm import FORMATS, assert_close, make, run_gpu, run_ref
 
 pytestmark = pytest.mark.gpu
 
-TILES = [(16, 16), (32, 32), (32, 64), (64, 64), (128, 64), (128, 128), (192, 128)]
+TILES = [(16, 16), (32, 32), (32, 64), (64, 64), (128, 64), (128, 128), (192, 128), (96, 96)]
 NAN = float("nan")
 
 
@@ -96,3 +96,18 @@ def test_infinite_scales_and_special_codes(pkg, gpu):
         got = launch(pkg, d, M, N, K, "f32", "f32", True, 1 + i).float()
         assert torch.equal(torch.isnan(got), torch.isnan(want)), TILES[i]
         assert torch.equal(torch.isinf(got), torch.isinf(want)), TILES[i]
+
+
+@pytest.mark.parametrize("afmt,bfmt,col", FORMATS)
+@pytest.mark.parametrize("M,N", [(97, 400), (95, 1104), (192, 96), (50, 208)])
+def test_96_column_tiles_straddle_weight_blocks(pkg, gpu, M, N, afmt, bfmt, col):
+    # Tiles from columns 96, 192, 288 and 384: their waves of 48 columns meet the
+    # 128-column boundaries after 0 to 3 of their 16-column tiles; N ends a tile
+    # inside a wave, in its first block and past its last.
+    K = 896
+    note(f"gemm 96 x 96 tile M={M} N={N} a={afmt} b={bfmt} col={col}")
+    ops = make(M, N, K, afmt, bfmt, col, seed=M + N)
+    d = [t.to(gpu).contiguous() for t in ops]
+    want = launch(pkg, d, M, N, K, afmt, bfmt, col, 256)
+    got = launch(pkg, d, M, N, K, afmt, bfmt, col, 1 + TILES.index((96, 96)))
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
