@@ -79,7 +79,7 @@ def pyext_path() -> Path:
 
 def pyext_command() -> list[str]:
     """g++ line of the CPython binding (csrc/fagq_py.cpp) against torch's headers.
-    Host code only: it calls fagq_launch through a pointer it is handed at import."""
+    Host code only: it calls the library through pointers it is handed at import."""
     import sysconfig
     import torch
     from torch.utils import cpp_extension

@@ -804,7 +804,7 @@ int check_args(const void* q, const void* c_kv, const void* out, const void* dou
   return FAGQ_OK;
 }
 
-// Overlap checks with the workspace, the device check and the three launches.
+// Overlap checks with the workspace, the device check and the launches.
 int launch(const void* q, const void* c_kv, const void* out, const void* dout, const float* lse,
            void* dq, void* dc_kv, void* workspace, int64_t need, int64_t B, int64_t H, int64_t S,
            int64_t D, float sm_scale, int dq_dtype, int dc_dtype, void* stream) {
