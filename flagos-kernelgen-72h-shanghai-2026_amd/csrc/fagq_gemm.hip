@@ -571,8 +571,13 @@ using Ring128x64 = Ring<2, 2, 4, 2, 3>;      // two workgroups per CU
 using Ring128x128 = Ring<2, 4, 4, 2, 3>;
 using Ring192x128 = Ring<3, 4, 4, 2, 4>;
 using Ring96x96 = Ring<3, 3, 2, 2, 3>;       // two workgroups per CU
-// The same for one round of 256-row tiles, 256 and 192 columns wide.
-constexpr double kPP256C = 13.0, kPP256T = 1.368, kPP192C = 6.87, kPP192T = 0.923;
+// The same for one round of 256-row tiles, 256 and 192 columns wide.  The 192-wide
+// line is that of nearly full rounds (100 .. 250 workgroups), where the choice is
+// close: of 55 shapes at the line's two sides those it gives to a small tile (23,
+// K <= 2304) run 8.6 % faster there than in 256 x 192 (geometric mean; 5 % or more for
+// most, 0.3 % slower at worst), and those with larger K that stay run up to 10 %
+// slower in a small tile.
+constexpr double kPP256C = 13.0, kPP256T = 1.368, kPP192C = 10.5, kPP192T = 0.86;
 constexpr int64_t kSmallMinBlocks = 4;       // k-blocks: the fits' range ends at K = 512
 constexpr int64_t kSmallMaxK = 1 << 16;      // row offsets of 192 rows stay far below 2^31
 constexpr int64_t kSmallMaxRows = 1 << 16;   // M and N of a forced small tile: a call's own reach
