@@ -150,8 +150,9 @@ _fast_tried = False
 
 def fast_launch():
     """launch() of the CPython binding (csrc/fagq_py.cpp), bound to this
-    process's libfagq.so, or None when that module is not built or does not
-    import (the ctypes path then serves every call; both reach fagq_launch)."""
+    process's libfagq.so, or None when that module is not built, does not import
+    or is an older build without an entry this layer binds (the ctypes path then
+    serves every call; both reach fagq_launch)."""
     global _fast, _fast_mod, _fast_tried
     if _fast_tried:
         return _fast
@@ -168,8 +169,8 @@ def fast_launch():
                                      lib.fagq_mla_bwd_launch)])
                 _fast = _fagq_py.launch
                 _fast_mod = _fagq_py
-            except ImportError:
-                _fast = None
+            except (ImportError, AttributeError):
+                _fast = _fast_mod = None
             _fast_tried = True
     return _fast
 

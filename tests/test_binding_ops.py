@@ -39,3 +39,18 @@ def test_cpu_tensors_and_odd_arguments_are_left_to_python(mod):
 def test_fast_module_needs_a_plain_gpu_tensor(mod):
     for t in (torch.zeros(2), None, torch.nn.Parameter(torch.zeros(2)), torch.zeros(2, device="meta")):
         assert mod.fast_module(t) == (None, None)
+
+
+def test_an_older_binding_leaves_every_call_to_ctypes(pkg, monkeypatch):
+    """A _fagq_py built before an entry was added has bind() but not bind_all()."""
+    import sys
+    import types
+    from fagq_mi355x import _lib
+    old = types.ModuleType("fagq_mi355x._fagq_py")
+    old.bind, old.launch = (lambda *a: None), (lambda *a: 0)
+    monkeypatch.setitem(sys.modules, "fagq_mi355x._fagq_py", old)
+    monkeypatch.setattr(pkg, "_fagq_py", old, raising=False)
+    for name, v in (("_fast", None), ("_fast_mod", None), ("_fast_tried", False)):
+        monkeypatch.setattr(_lib, name, v)
+    assert _lib.fast_launch() is None
+    assert _lib._fast is None and _lib._fast_mod is None and _lib._fast_tried
