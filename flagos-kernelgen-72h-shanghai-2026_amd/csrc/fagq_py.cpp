@@ -16,12 +16,14 @@
 //               0 = RNE, 1 = truncation, anything else = invalid.
 //     Returns fagq_launch's status, or kArgError when a tensor argument is
 //     rejected here (the Python layer then raises its detailed error).
-//   quant(...), parts(...), gemm(...), dsa(...), mla(...): the other operators,
-//     allocation included.  They return the outputs (dsa and mla: 0), the
-//     library's status as an int where it is an error, or kArgError for any
-//     argument that the Python layer should look at: it then takes the call from
-//     the start, with the same results and its own wording of the errors.
-//     Nothing is allocated or launched before all arguments are accepted.
+//   quant(...) (with a list of tensors the multi-input form), gemm(...), dsa(...),
+//     mla(...): the other operators, allocation included.  They return the outputs
+//     (dsa and mla: 0), the library's status as an int where it is an error, or
+//     kArgError for any argument that the Python layer should look at: it then takes
+//     the call from the start, with the same results and its own wording of the errors.
+//     Nothing is allocated or launched before all arguments are accepted.  The
+//     allocations (which may reach hipMalloc, or wait for the device to free cached
+//     blocks) and the launch run without the GIL, as torch's and ctypes' own calls do.
 //
 // In all of them the caller passes the current stream of the tensors' device
 // and has made that device current.
@@ -183,6 +185,17 @@ PyObject* launch(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 
 PyObject* arg_error() { return PyLong_FromLong(kArgError); }
 
+// Releases the GIL for its scope, also when an exception leaves it.  The argument
+// objects outlive the call (the caller's frame holds them); their data pointers
+// are read before.
+struct NoGil {
+  PyThreadState* const state = PyEval_SaveThread();
+  NoGil() = default;
+  NoGil(const NoGil&) = delete;
+  NoGil& operator=(const NoGil&) = delete;
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+
 // Plain tensors only: a subclass may override what the Python layer calls.
 bool is_plain(PyObject* o) { return THPVariable_CheckExact(o); }
 
@@ -219,11 +232,11 @@ bool stream_arg(PyObject* o, void** out) {
 }
 
 // Code and scale tensors of the functional forms.
-at::Tensor empty_codes(const at::Tensor& x, int64_t M, int64_t D, bool fp8) {
-  return at::empty({M, D}, at::TensorOptions(x.device()).dtype(fp8 ? at::kFloat8_e4m3fn : at::kChar));
+at::Tensor empty_codes(c10::Device device, int64_t M, int64_t D, bool fp8) {
+  return at::empty({M, D}, at::TensorOptions(device).dtype(fp8 ? at::kFloat8_e4m3fn : at::kChar));
 }
-at::Tensor empty_scale(const at::Tensor& x, int64_t M, int64_t groups, bool ue8m0, bool col_major) {
-  const auto o = at::TensorOptions(x.device()).dtype(ue8m0 ? at::kByte : at::kFloat);
+at::Tensor empty_scale(c10::Device device, int64_t M, int64_t groups, bool ue8m0, bool col_major) {
+  const auto o = at::TensorOptions(device).dtype(ue8m0 ? at::kByte : at::kFloat);
   return col_major ? at::empty_strided({M, groups}, {1, M}, o) : at::empty({M, groups}, o);
 }
 
@@ -290,31 +303,42 @@ PyObject* quant(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int sf = ue ? FAGQ_SCALE_UE8M0 : FAGQ_SCALE_F32;
   const int64_t groups = D / G;
 
-  const at::Tensor residual_out = inplace ? residual : at::empty_like(residual);
-  const at::Tensor q = empty_codes(x, M, D, fp8);
-  const at::Tensor scale = empty_scale(x, M, groups, ue, col);
-  if (M != 0) {
-    // A [M, groups] tensor with one row or column is both: row-major, as in Python.
-    const int layout = scale.is_contiguous() ? FAGQ_LAYOUT_ROW_MAJOR : FAGQ_LAYOUT_COL_MAJOR;
-    const float eps = (float)PyFloat_AS_DOUBLE(args[3]);
-    int st;
-    if (multi) {
-      const void* ptrs[FAGQ_MAX_PARTS];
-      for (Py_ssize_t i = 0; i < n; ++i) ptrs[i] = THPVariable_Unpack(xs[i]).data_ptr();
-      st = g_parts(ptrs, (int)n, residual.data_ptr(), weight.data_ptr(), residual_out.data_ptr(),
-                   q.data_ptr(), scale.data_ptr(), M, D, G, eps, qf, sf, layout, rnd, stream);
-    } else if (act == FAGQ_DT_BF16 && res == FAGQ_DT_BF16) {
-      st = g_launch(x.data_ptr(), residual.data_ptr(), weight.data_ptr(), residual_out.data_ptr(),
-                    nullptr, q.data_ptr(), scale.data_ptr(), M, D, G, eps, qf, sf, layout, rnd,
-                    stream);
-    } else {
-      st = g_launch_typed(x.data_ptr(), residual.data_ptr(), weight.data_ptr(),
-                          residual_out.data_ptr(), nullptr, q.data_ptr(), scale.data_ptr(), M, D,
-                          G, eps, qf, sf, layout, rnd, act, res, stream);
-      if (st == FAGQ_E_FORMAT) return arg_error();       // a type pair the library refuses
-    }
-    if (st != FAGQ_OK) return PyLong_FromLong(st);
+  // The list is the caller's to change once the GIL is released: its tensors are held.
+  at::Tensor held[FAGQ_MAX_PARTS];
+  const void* ptrs[FAGQ_MAX_PARTS];
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    const at::Tensor& t = THPVariable_Unpack(xs[i]);
+    if (multi) held[i] = t;
+    ptrs[i] = t.data_ptr();
   }
+  const void* const rp = residual.data_ptr();
+  const void* const wp = weight.data_ptr();
+  const float eps = (float)PyFloat_AS_DOUBLE(args[3]);
+  const c10::Device device = x.device();
+  at::Tensor residual_out, q, scale;
+  int st = FAGQ_OK;
+  {
+    NoGil no_gil;
+    residual_out = inplace ? residual : at::empty_like(residual);
+    q = empty_codes(device, M, D, fp8);
+    scale = empty_scale(device, M, groups, ue, col);
+    if (M != 0) {
+      // A [M, groups] tensor with one row or column is both: row-major, as in Python.
+      const int layout = scale.is_contiguous() ? FAGQ_LAYOUT_ROW_MAJOR : FAGQ_LAYOUT_COL_MAJOR;
+      if (multi)
+        st = g_parts(ptrs, (int)n, rp, wp, residual_out.data_ptr(), q.data_ptr(), scale.data_ptr(),
+                     M, D, G, eps, qf, sf, layout, rnd, stream);
+      else if (act == FAGQ_DT_BF16 && res == FAGQ_DT_BF16)
+        st = g_launch(ptrs[0], rp, wp, residual_out.data_ptr(), nullptr, q.data_ptr(),
+                      scale.data_ptr(), M, D, G, eps, qf, sf, layout, rnd, stream);
+      else
+        st = g_launch_typed(ptrs[0], rp, wp, residual_out.data_ptr(), nullptr, q.data_ptr(),
+                            scale.data_ptr(), M, D, G, eps, qf, sf, layout, rnd, act, res, stream);
+    }
+  }
+  // A type pair the library refuses goes to the Python checks.
+  if (st == FAGQ_E_FORMAT && !(act == FAGQ_DT_BF16 && res == FAGQ_DT_BF16)) return arg_error();
+  if (st != FAGQ_OK) return PyLong_FromLong(st);
   return three(residual_out, q, scale);   // inplace: the caller's own tensor object
   END_HANDLE_TH_ERRORS
 }
@@ -357,10 +381,16 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   else if (as.stride(0) == 1 && as.stride(1) == M) layout = FAGQ_LAYOUT_COL_MAJOR;
   else return arg_error();
   if (has_out && !rows_ok(THPVariable_Unpack(args[4]), cshape, dev, at::kBFloat16)) return arg_error();
-  const at::Tensor out = has_out ? THPVariable_Unpack(args[4])
-                                 : at::empty({M, N}, at::TensorOptions(a.device()).dtype(at::kBFloat16));
-  const int st = g_gemm(a.data_ptr(), as.data_ptr(), b.data_ptr(), bs.data_ptr(), out.data_ptr(), M,
-                        N, K, asf, layout, bsf, stream);
+  const void* const p[4] = {a.data_ptr(), as.data_ptr(), b.data_ptr(), bs.data_ptr()};
+  const c10::Device device = a.device();
+  at::Tensor out;
+  if (has_out) out = THPVariable_Unpack(args[4]);
+  int st;
+  {
+    NoGil no_gil;
+    if (!has_out) out = at::empty({M, N}, at::TensorOptions(device).dtype(at::kBFloat16));
+    st = g_gemm(p[0], p[1], p[2], p[3], out.data_ptr(), M, N, K, asf, layout, bsf, stream);
+  }
   if (st != FAGQ_OK) return PyLong_FromLong(st);
   return THPVariable_Wrap(out);
   END_HANDLE_TH_ERRORS
@@ -398,9 +428,15 @@ PyObject* dsa(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       !rows_ok(*t[2], at::IntArrayRef(kv, 1), dev, it) || !rows_ok(*t[3], ob, dev, at::kInt) ||
       !rows_ok(*t[4], ob, dev, at::kInt))
     return arg_error();
-  return PyLong_FromLong(g_dsa(s.data_ptr(), sdt, t[0]->data_ptr(), t[1]->data_ptr(),
-                               t[2]->data_ptr(), it == at::kLong ? FAGQ_DSA_I64 : FAGQ_DSA_I32,
-                               t[3]->data_ptr(), t[4]->data_ptr(), B, H, Q, NB, bs, k, stream));
+  void* p[6] = {s.data_ptr()};
+  for (int i = 0; i < 5; ++i) p[1 + i] = t[i]->data_ptr();
+  int st;
+  {
+    NoGil no_gil;
+    st = g_dsa(p[0], sdt, p[1], p[2], p[3], it == at::kLong ? FAGQ_DSA_I64 : FAGQ_DSA_I32, p[4],
+               p[5], B, H, Q, NB, bs, k, stream);
+  }
+  return PyLong_FromLong(st);
   END_HANDLE_TH_ERRORS
 }
 
@@ -438,12 +474,18 @@ PyObject* mla(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     return arg_error();
   const int64_t need = g_mla_bytes(B, S, D);
   if (need < 0) return arg_error();
-  const at::Tensor ws = at::empty({std::max<int64_t>(need, 16)},
-                                  at::TensorOptions(t[0]->device()).dtype(at::kByte));
-  return PyLong_FromLong(g_mla(t[0]->data_ptr(), t[1]->data_ptr(), t[2]->data_ptr(),
-                               t[3]->data_ptr(), static_cast<const float*>(t[4]->data_ptr()),
-                               t[5]->data_ptr(), t[6]->data_ptr(), ws.data_ptr(), ws.numel(), B, H,
-                               S, D, (float)sm_scale, dq, dc, stream));
+  void* p[7];
+  for (int i = 0; i < 7; ++i) p[i] = t[i]->data_ptr();
+  const c10::Device device = t[0]->device();
+  int st;
+  {
+    NoGil no_gil;
+    const at::Tensor ws = at::empty({std::max<int64_t>(need, 16)},
+                                    at::TensorOptions(device).dtype(at::kByte));
+    st = g_mla(p[0], p[1], p[2], p[3], static_cast<const float*>(p[4]), p[5], p[6], ws.data_ptr(),
+               ws.numel(), B, H, S, D, (float)sm_scale, dq, dc, stream);
+  }
+  return PyLong_FromLong(st);
   END_HANDLE_TH_ERRORS
 }
 

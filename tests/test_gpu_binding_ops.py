@@ -174,3 +174,76 @@ def test_other_streams_and_threads(pkg, gpu):
     [t.start() for t in ts]
     [t.join() for t in ts]
     assert not bad
+
+
+HOLD_C = """
+#include <unistd.h>
+long long hold(void) { usleep(150000); return 0; }
+"""
+
+
+def test_launches_leave_the_gil_to_other_threads(pkg, gpu, tmp_path):
+    """The library's entry points replaced by one that takes 150 ms on the host: a
+    Python thread beside the call runs on (it would not get a turn under the GIL)."""
+    import ctypes
+    import shutil
+    import subprocess
+    import threading
+    import time
+    from fagq_mi355x import _lib
+    from fagq_mi355x.workloads import MlaWorkload, make_mla_inputs
+    cc = shutil.which("gcc") or shutil.which("cc")
+    if cc is None:
+        pytest.skip("no C compiler")
+    note("binding without the GIL")
+    (tmp_path / "hold.c").write_text(HOLD_C)
+    subprocess.run([cc, "-shared", "-fPIC", "-o", str(tmp_path / "hold.so"), str(tmp_path / "hold.c")],
+                   check=True)
+    addr = lambda f: ctypes.cast(f, ctypes.c_void_p).value
+    hold = addr(ctypes.CDLL(str(tmp_path / "hold.so")).hold)
+    assert _lib.fast_launch() is not None
+    mod, lib = _lib._fast_mod, _lib.load()
+    z = lambda *s, dt=BF16: torch.zeros(*s, dtype=dt, device=gpu)
+    x, w = z(4, 256), z(256)
+    i32 = lambda *s: z(*s, dt=torch.int32)
+    q, c, out, do, lse = (t.to(gpu) for t in make_mla_inputs(MlaWorkload("t", 1, 2, 20, 64)))
+    dq, dc = torch.empty_like(q), torch.empty_like(c)
+    calls = {
+        "quant": lambda: pkg.fused_add_rmsnorm_group_quant_fn(x, x, w),
+        "typed": lambda: pkg.fused_add_rmsnorm_group_quant_fn(x.half(), x.half(), w.half()),
+        "parts": lambda: pkg.fused_reduce_add_rmsnorm_group_quant([x, x], x, w),
+        "gemm": lambda: pkg.fp8_block_scaled_gemm(z(4, 128, dt=FP8), z(4, 1, dt=F32),
+                                                  z(16, 128, dt=FP8), z(1, 1, dt=F32)),
+        "dsa": lambda: pkg.dsa_topk_page_table_transform(z(1, 1, 2, 64, dt=F32), i32(1, 64), i32(1, 2),
+                                                         i32(1), i32(1, 1, 2, 8), i32(1, 1, 2, 8), 16, 8),
+        "mla": lambda: pkg.mla_bwd_nope_dkdv(q, c, out, do, lse, dq, dc, 0.1),
+    }
+    for f in calls.values():                              # first calls, on the library itself
+        f()
+    torch.cuda.synchronize()
+    ticks, stop = [0], threading.Event()
+
+    def tick():
+        while not stop.is_set():
+            ticks[0] += 1
+            time.sleep(0.001)
+    t = threading.Thread(target=tick)
+    t.start()
+    got = {}
+    try:
+        mod.bind(hold, hold)
+        mod.bind_all(hold, hold, hold, addr(lib.fagq_mla_bwd_workspace_bytes), hold)
+        for name, f in calls.items():
+            t0, n0 = time.perf_counter(), ticks[0]
+            f()
+            got[name] = (ticks[0] - n0, time.perf_counter() - t0)
+    finally:
+        mod.bind(addr(lib.fagq_launch), addr(lib.fagq_launch_typed))
+        mod.bind_all(*[addr(f) for f in (lib.fagq_launch_parts, lib.fagq_gemm_launch,
+                                         lib.fagq_dsa_topk_launch, lib.fagq_mla_bwd_workspace_bytes,
+                                         lib.fagq_mla_bwd_launch)])
+        stop.set()
+        t.join()
+    for name, (n, s) in got.items():
+        # 150 sleeps of 1 ms fit; a thread kept out has its one turn at either end.
+        assert s >= 0.15 and n >= 20, (name, got)
