@@ -237,7 +237,9 @@ at::Tensor empty_codes(c10::Device device, int64_t M, int64_t D, bool fp8) {
 }
 at::Tensor empty_scale(c10::Device device, int64_t M, int64_t groups, bool ue8m0, bool col_major) {
   const auto o = at::TensorOptions(device).dtype(ue8m0 ? at::kByte : at::kFloat);
-  return col_major ? at::empty_strided({M, groups}, {1, M}, o) : at::empty({M, groups}, o);
+  // The strides of empty({groups, M}).t(), which are at least 1 where M is 0.
+  return col_major ? at::empty_strided({M, groups}, {1, std::max<int64_t>(M, 1)}, o)
+                   : at::empty({M, groups}, o);
 }
 
 PyObject* three(const at::Tensor& a, const at::Tensor& b, const at::Tensor& c) {

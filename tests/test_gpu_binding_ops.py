@@ -48,6 +48,9 @@ QUANT = [dict(M=4, D=8192, out_dtype=I8), dict(M=1, D=128, scale_col_major=True)
          dict(M=5, D=512, out_dtype=I8, rounding=None), dict(M=5, D=512, out_dtype=I8, rounding="trunc"),
          dict(M=7, D=768, rounding="trunc"), dict(M=9, D=512, act=F16, res=F16, scale_col_major=True),
          dict(M=9, D=512, res=F32), dict(M=9, D=512, act=F32, res=F32), dict(M=0, D=256),
+         dict(M=0, D=256, scale_col_major=True), dict(M=0, D=0), dict(M=0, D=0, scale_col_major=True),
+         dict(M=3, D=0), dict(M=0, D=192, group_size=96), dict(M=0, D=256, eps=-1.0),
+         dict(M=0, D=256, act=F32, res=BF16),
          dict(M=6, D=512, inplace_residual=True),
          # what the Python layer refuses or the library does
          dict(M=4, D=512, act=F32, res=BF16), dict(M=4, D=512, group_size=96), dict(M=4, D=512, group_size=32),
