@@ -55,6 +55,11 @@ class GemmRoute(ctypes.Structure):
                 ("grid_blocks", ctypes.c_int64)]
 
 
+class MlaRoute(ctypes.Structure):
+    _fields_ = [("dims", ctypes.c_int32), ("tile_dims", ctypes.c_int32),
+                ("heads_in_flight", ctypes.c_int32), ("head_planes", ctypes.c_int32)]
+
+
 SIGNATURES = {
     "fagq_launch": ([_P] * 7 + [_I64, _I64, _I64, _F, _I, _I, _I, _I, _P], _I),
     "fagq_launch_typed": ([_P] * 7 + [_I64, _I64, _I64, _F, _I, _I, _I, _I, _I, _I, _P], _I),
@@ -72,6 +77,7 @@ SIGNATURES = {
     "fagq_gemm_launch_mapped": ([_P] * 5 + [_I64, _I64, _I64, _I, _I, _I, _I, _P], _I),
     "fagq_gemm_query_route": ([_I64, _I64, _I64, ctypes.POINTER(GemmRoute)], _I),
     "fagq_mla_bwd_workspace_bytes": ([_I64, _I64, _I64], _I64),
+    "fagq_mla_bwd_query_route": ([_I64] * 4 + [_I, _I64, ctypes.POINTER(MlaRoute)], _I),
     "fagq_mla_bwd_launch": ([_P] * 8 + [_I64] * 5 + [_F, _I, _I, _P], _I),
     "fagq_mla_bwd_launch_noalloc": ([_P] * 7 + [_I64] * 4 + [_F, _I, _I, _P], _I),
 }
@@ -224,6 +230,14 @@ def query_route(M: int, D: int, group_size: int, scale_format: int = SCALE_F32,
         check(load().fagq_query_route_typed(M, D, group_size, scale_format, scale_layout, act, res,
                                             ctypes.byref(r)), "fagq_query_route_typed")
     return {f: getattr(r, f) for f, _ in Route._fields_ if f != "reserved"}
+
+
+def query_mla_route(B: int, H: int, S: int, D: int, dq_f32: bool, slice: int = 0) -> dict:
+    """How fagq_mla_bwd_launch runs a column slice of a shape (include/fagq_diag.h)."""
+    r = MlaRoute()
+    check(load().fagq_mla_bwd_query_route(B, H, S, D, 0 if dq_f32 else 1, slice, ctypes.byref(r)),
+          "fagq_mla_bwd_query_route")
+    return {f: getattr(r, f) for f, _ in MlaRoute._fields_}
 
 
 def query_route_parts(M: int, D: int, group_size: int, nparts: int,

@@ -8,14 +8,17 @@
 //   rows i >= E: dq_i = scale * do_i
 //   dc_j = sum_{i >= j} hs_i / (i + 1), hs_i = sum_h do[h, i]
 //
-// Kernels, in stream order.  Long sequences (see is_short):
+// Kernels, in stream order.  The long form (see pick_form):
 //   K1 mla_stream_do   - the one pass over dO (all the HBM traffic): per row
 //                        and all H heads, dq = scale * do (rows >= E) and the
 //                        head sum, stored as hs_i / (i + 1) in the workspace.
 //                        A lane owns 8 consecutive dims (16-byte loads), a
 //                        workgroup 2048 / D rows, so each head contributes a
 //                        contiguous 4 KB (D = 512) segment per workgroup.
-//   K2 mla_block_totals - per block of 16-64 rows: fp32 totals of hs / (i + 1).
+//                        With two head planes each half of the heads is a
+//                        workgroup of its own, with its own plane of sums.
+//   K2 mla_block_totals - per block of 16-64 rows: fp32 totals of hs / (i + 1);
+//                        two planes are added here, the sum into the first.
 //   K3 mla_exact_rows_suffix_scan - one launch of 1024-thread workgroups, two
 //                        kinds:
 //                        * exact rows, one per (b, h): q, do and c rows 0..E-1
@@ -31,8 +34,8 @@
 //                        runs them in the part of the chip those leave idle.
 // K2 and K3 issue each thread's loads as one batch: at these sizes they are
 // latency-bound: every dependent round trip to memory adds its full latency.
-// Short sequences, two launches: mla_short_do (the dO pass with the running
-// sums of 8-row blocks, and the exact rows) and mla_short_scan.
+// The short form, two launches: mla_short_do (the dO pass with the running sums
+// of 8-row blocks, and the exact rows) and mla_short_scan.
 //
 // D above kSliceD (512) runs as column slices of at most kSliceD dims: K1, the
 // block totals and K3 are per column, so each slice runs them on its columns
@@ -44,8 +47,10 @@
 
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 #include "fagq.h"
+#include "fagq_diag.h"
 #include "fagq_dispatch.hpp"
 #include "fagq_mla.h"
 
@@ -68,9 +73,11 @@ struct MArgs {
   const float* lse;
   void* dq;
   void* dc;
-  float* hs;          // workspace: [B, S, D] head sums / (i + 1); for short sequences their
-                      // reverse running sums within blocks of kBlockRows rows
+  float* hs;          // workspace: [planes, B, S, D] head sums / (i + 1); in the short form
+                      // their reverse running sums within blocks of kBlockRows rows
   float* tot;         // workspace: [B, nblk, D] block totals
+  int64_t hs_plane;   // elements between the planes (B * S * D)
+  int32_t planes;     // 1, or 2: the heads' halves, each with its plane
   int32_t brows;      // rows per scan block
   int32_t nblk;       // ceil(S / brows)
   int32_t H, S;
@@ -187,12 +194,19 @@ __device__ __forceinline__ void stream_heads(const MArgs& g, int b, int row, uin
   }
 }
 
-// K1.  grid (ceil(S / rows_per_wg), B); rows_per_wg = 256 / (D / 8).  U heads'
-// loads are in flight per lane: U = 2 with bf16 dq (50 VGPRs, 8 workgroups per
-// CU) and U = 1 with fp32 dq, whose stores are twice the loads' bytes (2 B / 4
+// The heads of a plane: [h0, h1), never empty (two planes have 40 heads or more).
+__device__ __forceinline__ void plane_heads(const MArgs& g, int plane, int& h0, int& h1) {
+  const int hpp = (g.H + g.planes - 1) >> (g.planes - 1);
+  h0 = plane * hpp;
+  h1 = h0 + hpp < g.H ? h0 + hpp : g.H;
+}
+
+// K1.  grid (ceil(S / rows_per_wg), B, planes); rows_per_wg = 256 / (D / 8).  U
+// heads' loads are in flight per lane: U = 2 with bf16 dq (50 VGPRs, 8 workgroups
+// per CU) and U = 1 with fp32 dq, whose stores are twice the loads' bytes (2 B / 4
 // B, 2 x 64 x 4096 x 512: 297 against 308 us for the pass; 2 x 64 x 1900 x 512
 // 147.9 us per call against 157.2 with U = 8); U = 8 (110 VGPRs, 4 per CU) with
-// bf16 dq for grids that fit 4 per CU.
+// bf16 dq for grids that fit 4 per CU (figures: pick_form).
 template <int U, bool HALVES>
 __global__ void __launch_bounds__(kThreads) mla_stream_do(const MArgs g) {
   const int lpr = g.D / 8;                        // lanes per row
@@ -212,13 +226,15 @@ __global__ void __launch_bounds__(kThreads) mla_stream_do(const MArgs g) {
   const uint32_t wa = (uint32_t)row * (uint32_t)g.D + lo;
   const uint32_t half = (uint32_t)g.D / 2u;
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  stream_heads<U, HALVES>(g, b, row, ea, ea + half, 0, g.H, acc);
+  int h0, h1;
+  plane_heads(g, (int)blockIdx.z, h0, h1);
+  stream_heads<U, HALVES>(g, b, row, ea, ea + half, h0, h1, acc);
   const float n1 = (float)(row + 1);
   float o[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) o[k] = acc[k] / n1;
   const uint32_t sd = (uint32_t)g.S * (uint32_t)g.D;
-  const rsrc_t rhs = make_rsrc(g.hs + (int64_t)b * sd, sd * 4u);
+  const rsrc_t rhs = make_rsrc(g.hs + (int64_t)blockIdx.z * g.hs_plane + (int64_t)b * sd, sd * 4u);
   store_lane<HALVES>(rhs, false, wa, wa + half, o);
 }
 
@@ -413,27 +429,39 @@ struct Parts {
 };
 
 // Totals of block blk (g.brows rows) of batch b: part p of the block's threads
-// sums rows r0 + p, r0 + p + np, ..., kBatch of them loaded together; the parts'
-// totals are joined in LDS, in part order.
+// sums rows r0 + p, r0 + p + np, ..., kBatch / PL of them loaded together; the
+// parts' totals are joined in LDS, in part order.  PL 2: each row's two planes are
+// added, and the sum written over the first, the only one that K3 reads.
+template <int PL>
 __device__ __forceinline__ void block_total(const MArgs& g, int b, int blk) {
+  constexpr int R = kBatch / PL;
   extern __shared__ __align__(16) uint8_t smem[];
   float4* part = reinterpret_cast<float4*>(smem);
   const Parts P(g.D);
   const int r0 = blk * g.brows;
   const int r1 = r0 + g.brows < g.S ? r0 + g.brows : g.S;
-  const float* __restrict__ hs = g.hs + (int64_t)b * g.S * g.D + 4 * P.col;
+  float* __restrict__ hs = g.hs + (int64_t)b * g.S * g.D + 4 * P.col;
   float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
   if (P.p < P.np) {
-    for (int r = r0 + P.p; r < r1; r += kBatch * P.np) {
-      float4 v[kBatch];
+    for (int r = r0 + P.p; r < r1; r += R * P.np) {
+      float4 v[R][PL];
 #pragma unroll
-      for (int i = 0; i < kBatch; ++i) {
-        const int rr = r + i * P.np < r1 ? r + i * P.np : r0;
-        v[i] = *reinterpret_cast<const float4*>(hs + (int64_t)rr * g.D);
+      for (int i = 0; i < R; ++i) {
+        // Clamped to a row that no other thread writes (PL 2); r0 is one load for all.
+        const int rr = r + i * P.np < r1 ? r + i * P.np : PL == 2 ? r : r0;
+#pragma unroll
+        for (int p = 0; p < PL; ++p)
+          v[i][p] = *reinterpret_cast<const float4*>(hs + p * g.hs_plane + (int64_t)rr * g.D);
       }
 #pragma unroll
-      for (int i = 0; i < kBatch; ++i)
-        if (r + i * P.np < r1) add4(a, v[i]);
+      for (int i = 0; i < R; ++i) {
+        if (r + i * P.np >= r1) continue;
+        if constexpr (PL == 2) {
+          add4(v[i][0], v[i][1]);
+          *reinterpret_cast<float4*>(hs + (int64_t)(r + i * P.np) * g.D) = v[i][0];
+        }
+        add4(a, v[i][0]);
+      }
     }
   }
   part[threadIdx.x] = a;
@@ -445,8 +473,9 @@ __device__ __forceinline__ void block_total(const MArgs& g, int b, int blk) {
 }
 
 // grid (nblk, B)
+template <int PL>
 __global__ void __launch_bounds__(kWide) mla_block_totals(const MArgs g) {
-  block_total(g, (int)blockIdx.y, (int)blockIdx.x);
+  block_total<PL>(g, (int)blockIdx.y, (int)blockIdx.x);
 }
 
 // ------------------------------------------------------------------ K3
@@ -537,10 +566,12 @@ __global__ void __launch_bounds__(kWide) mla_exact_rows_suffix_scan(const MArgs 
 // the block's reverse running sums (with the 1 / (i + 1)) go to the workspace,
 // whose rows 0, 8, 16, .. then are the blocks' totals.  One launch replaces a
 // pass that wrote up to 8 partial planes and a kernel for the totals, and the
-// last one only adds the later blocks' totals.  The exact rows, which depend on
-// nothing else, are the grid's first workgroups and run beside the dO pass.
-// Bound by the dO pass's bytes, and below about 20 us by the two launches'
-// latency (figures: short_tile).
+// last one only adds the later blocks' totals.  With two planes each half of the
+// heads is a workgroup of its own: few tiles of many heads leave CUs idle, and a
+// wave's chain of heads is long.  The exact rows, which depend on nothing else,
+// are the grid's first workgroups and run beside the dO pass.  Bound by the dO
+// pass's bytes, and below about 20 us by the two launches' latency (figures:
+// pick_form).
 constexpr int kBlockRows = 8;
 constexpr int kShortWaves = 8;
 
@@ -560,14 +591,17 @@ __global__ void __launch_bounds__(64 * kShortWaves) mla_short_do(const MArgs g) 
   const int t = threadIdx.x, lane = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
   const int rw = w % RW, hg = w / RW;
-  const int x = (int)blockIdx.x - g.nexact;
+  const int y = (int)blockIdx.x - g.nexact;
+  const int plane = y & (g.planes - 1), x = y >> (g.planes - 1);
   const int ncol = g.D / CW, ct = x % ncol, blk = x / ncol;   // CW divides D
   const int r0 = blk * kBlockRows;
   const int brow = rw * WR + lane / LPR, row = r0 + brow;     // the lane's row in the block, of S
   const int li = lane % LPR;
-  const int hps = (g.H + HG - 1) / HG;
-  const int hbeg = hg * hps < g.H ? hg * hps : g.H;
-  const int hend = hbeg + hps < g.H ? hbeg + hps : g.H;
+  int h0, h1;
+  plane_heads(g, plane, h0, h1);
+  const int hps = (h1 - h0 + HG - 1) / HG;
+  const int hbeg = h0 + hg * hps < h1 ? h0 + hg * hps : h1;
+  const int hend = hbeg + hps < h1 ? hbeg + hps : h1;
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (row < g.S && hbeg < hend) {
     const uint32_t ea = (uint32_t)row * (uint32_t)g.ld + (uint32_t)(ct * CW + li * (HALVES ? 4 : 8));
@@ -589,7 +623,7 @@ __global__ void __launch_bounds__(64 * kShortWaves) mla_short_do(const MArgs g) 
     float4 v[kBlockRows];
 #pragma unroll
     for (int k = 0; k < kBlockRows; ++k) v[k] = part[k * C4 + t];
-    float* const hs = g.hs + ((int64_t)b * g.S + r0) * g.D + ct * CW + 4 * t;
+    float* const hs = g.hs + plane * g.hs_plane + ((int64_t)b * g.S + r0) * g.D + ct * CW + 4 * t;
     float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int k = kBlockRows - 1; k >= 0; --k) {          // rows past S hold zeros
@@ -603,11 +637,29 @@ __global__ void __launch_bounds__(64 * kShortWaves) mla_short_do(const MArgs g) 
 // dc of a short sequence.  grid (nblk, B), g.brows rows each (a multiple of
 // kBlockRows): a row's dc is its running sum within its block of 8 rows plus
 // the totals of the later blocks.  Part p (see Parts) owns cr consecutive rows,
-// cr a power of two up to 8, so all in one block; it sums the totals of every
+// cr a power of two up to CR, so all in one block; it sums the totals of every
 // np-th block past the workgroup's rows, and after one barrier adds all parts'
-// sums, in part order, and the totals of the workgroup's own later blocks.
+// sums, in part order, and the totals of the workgroup's own later blocks.  PL 2:
+// every row and total is the sum of its two planes; both are loaded together, for
+// which the registers suffice where brows is 16 (CR 2, one later block).  Its sums
+// are kept in 64 bits until they are written: the planes' own roundings are two where
+// one plane has one (relative error of dc at 1 x 128 x 100 x 512: 5.2e-8; 7.0e-8 with sums in
+// 32 bits, 6.4e-8 with one plane).
+struct Sum64 {
+  double x, y, z, w;
+};
+__device__ __forceinline__ void add4(Sum64& a, const Sum64& b) {
+  a.x += b.x;
+  a.y += b.y;
+  a.z += b.z;
+  a.w += b.w;
+}
+template <int PL, int CR>
 __global__ void __launch_bounds__(kWide) mla_short_scan(const MArgs g) {
-  __shared__ float4 later[kWide];
+  constexpr int NEAR = CR == 2 ? 1 : kBlockRows - 1;     // later blocks in the workgroup's rows
+  constexpr int LB = kBlockRows / PL;                    // far totals loaded together
+  using Sum = std::conditional_t<PL == 2, Sum64, float4>;
+  __shared__ Sum later[kWide];
   const int b = (int)blockIdx.y;
   const Parts P(g.D);
   const int r0 = (int)blockIdx.x * g.brows;
@@ -619,48 +671,61 @@ __global__ void __launch_bounds__(kWide) mla_short_scan(const MArgs g) {
   const int nb = (g.S + kBlockRows - 1) / kBlockRows;    // blocks of 8 rows of the sequence
   const int next = (r0 + g.brows) / kBlockRows;          // the first past the workgroup's rows
   const float* __restrict__ hs = g.hs + (int64_t)b * g.S * g.D + 4 * P.col;
-  auto total = [&](int x) { return *reinterpret_cast<const float4*>(hs + (int64_t)x * kBlockRows * g.D); };
-  float4 rows[kBlockRows], near[kBlockRows];
-  float4 lat = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto load = [&](int row, float4 (&v)[PL]) {
+#pragma unroll
+    for (int p = 0; p < PL; ++p)
+      v[p] = *reinterpret_cast<const float4*>(hs + p * g.hs_plane + (int64_t)row * g.D);
+  };
+  auto add = [](Sum& a, const float4 (&v)[PL]) {
+    if constexpr (PL == 2)
+      add4(a, Sum64{(double)v[0].x + v[1].x, (double)v[0].y + v[1].y, (double)v[0].z + v[1].z,
+                    (double)v[0].w + v[1].w});
+    else
+      add4(a, v[0]);
+  };
+  float4 rows[CR][PL], near[NEAR][PL];
+  Sum lat = {0, 0, 0, 0};
   const int own = c0 / kBlockRows;                       // the block of the part's rows
-  const int nnear = (next < nb ? next : nb) - own - 1;   // later blocks of this workgroup, < 8
+  const int nnear = (next < nb ? next : nb) - own - 1;   // later blocks of this workgroup
   if (P.p < P.np && c0 < c1) {
 #pragma unroll
-    for (int k = 0; k < kBlockRows; ++k) {
-      if (k < cr) rows[k] = *reinterpret_cast<const float4*>(hs + (int64_t)(c0 + k < c1 ? c0 + k : c0) * g.D);
-      if (k < nnear) near[k] = total(own + 1 + k);
-    }
+    for (int k = 0; k < CR; ++k)
+      if (k < cr) load(c0 + k < c1 ? c0 + k : c0, rows[k]);
+#pragma unroll
+    for (int k = 0; k < NEAR; ++k)
+      if (k < nnear) load((own + 1 + k) * kBlockRows, near[k]);
   }
   if (P.p < P.np) {
-    for (int x = next + P.p; x < nb; x += kBlockRows * P.np) {
-      float4 v[kBlockRows];
+    for (int x = next + P.p; x < nb; x += LB * P.np) {
+      float4 v[LB][PL];
 #pragma unroll
-      for (int k = 0; k < kBlockRows; ++k) {
+      for (int k = 0; k < LB; ++k) {
         const int xx = x + k * P.np;
-        v[k] = total(xx < nb ? xx : x);
+        load((xx < nb ? xx : x) * kBlockRows, v[k]);
       }
 #pragma unroll
-      for (int k = 0; k < kBlockRows; ++k)
-        if (x + k * P.np < nb) add4(lat, v[k]);
+      for (int k = 0; k < LB; ++k)
+        if (x + k * P.np < nb) add(lat, v[k]);
     }
   }
   later[threadIdx.x] = lat;
   __syncthreads();
   if (P.p >= P.np || c0 >= c1) return;
-  float4 cy = make_float4(0.f, 0.f, 0.f, 0.f);
+  Sum cy = {0, 0, 0, 0};
   for (int q = 0; q < P.np; ++q) add4(cy, later[q * P.cpt + P.col]);
 #pragma unroll
-  for (int k = kBlockRows - 1; k >= 0; --k)
-    if (k < nnear) add4(cy, near[k]);
+  for (int k = NEAR - 1; k >= 0; --k)
+    if (k < nnear) add(cy, near[k]);
   float* __restrict__ dcf = static_cast<float*>(g.dc) + (int64_t)b * g.S * g.ld + 4 * P.col;
   uint16_t* __restrict__ dch = static_cast<uint16_t*>(g.dc) + (int64_t)b * g.S * g.ld + 4 * P.col;
   const bool bf16 = g.dc_bf16 != 0;
 #pragma unroll
-  for (int k = 0; k < kBlockRows; ++k) {
+  for (int k = 0; k < CR; ++k) {
     const int r = c0 + k;
     if (k < cr && r < c1) {
-      float4 o = cy;
-      add4(o, rows[k]);
+      Sum sum = cy;
+      add(sum, rows[k]);
+      const float4 o = make_float4((float)sum.x, (float)sum.y, (float)sum.z, (float)sum.w);
       if (bf16) {
         const uint2 wv = {pack_bf16x2(o.x, o.y), pack_bf16x2(o.z, o.w)};
         *reinterpret_cast<uint2*>(dch + (int64_t)r * g.ld) = wv;
@@ -687,55 +752,13 @@ int64_t k1_groups(int64_t B, int64_t S, int64_t D) {
   return ((S + rows_per_wg - 1) / rows_per_wg) * B;
 }
 
-// Planes of head sums the workspace is sized for.  The kernels use one; the
-// size that callers were told for a shape does not change.
+// Planes of head sums the workspace is sized for.  The kernels use one or two;
+// the size that callers were told for a shape does not change.
 int64_t workspace_planes(int64_t B, int64_t S, int64_t D) {
   if (D < 64) return 1;
   int64_t sp = 1;
   while (k1_groups(B, S, D) * sp < kMinK1Groups && sp < kMaxHeadSplit) sp *= 2;
   return sp;
-}
-
-// Column tile of the short sequences' dO pass: the widest with at least 320
-// workgroups, whose longer contiguous pieces of a row memory serves faster;
-// else 128 dims with all of a wave's 8 or more heads in flight, unless the grid
-// with the exact rows would put two workgroups on some CUs and one on others.
-// us per call in a replayed graph, H = 64, D = 512, bf16 gradients (B x S: the tile of
-// this rule, the others in the order 512 / 256 / 128 / 64): 1 x 300, fp32 gradients:
-// 128: 17.9, others 43.4 / 29.5 / - / 25.1; 2 x 256: 64: 24.0, 43.8 / 27.9 / 27.2; 2 x
-// 512: 128: 35.3, 50.2 / 40.6 / - / 42.7; 2 x 1024: 256: 60.0, 68.5 / - / 62.4 / 69.9;
-// 2 x 1900: 512: 102.2, - / 116.6 / 111.5 / 121.9.  Before this pass (partial planes,
-// block totals, scan with the exact rows): 25.6, 28.0, 38.9, 62.1 and 109.3.
-struct ShortTile {
-  const void* kernel;
-  int cw, head_groups;
-};
-template <int CW, int U>
-ShortTile make_short_tile(bool halves) {
-  return {halves ? reinterpret_cast<const void*>(&mla_short_do<CW, U, true>)
-                 : reinterpret_cast<const void*>(&mla_short_do<CW, U, false>),
-          CW, kShortWaves * 64 / (CW / 8) / kBlockRows};
-}
-ShortTile short_tile(int64_t B, int64_t S, int64_t ds, int64_t nexact, bool halves) {
-  const int64_t blocks = B * ((S + kBlockRows - 1) / kBlockRows);
-  if (ds % 512 == 0 && blocks * (ds / 512) >= 320) return make_short_tile<512, 4>(halves);
-  if (ds % 256 == 0 && blocks * (ds / 256) >= 320) return make_short_tile<256, 4>(halves);
-  if (ds % 128 == 0 && blocks * (ds / 128) >= 320) return make_short_tile<128, 4>(halves);
-  if (ds % 128 == 0 && blocks * (ds / 128) + B * nexact <= 320) return make_short_tile<128, 8>(halves);
-  return make_short_tile<64, 4>(halves);
-}
-
-// Sequences whose K1 has fewer than kMinK1Groups workgroups are short; with
-// fp32 dq, whose stores set the pass's rate, fewer than half of that (2 x 64 x
-// 1900 x 512: K1 with U = 1, 147.9 us, against 154.1 by the short pass; 2 x 64 x
-// 1024 x 512: 84.6 against 85.0).  Where only 64-dim tiles fit, few heads leave
-// their 8 head groups one or two heads each, and many such workgroups cost more
-// than K1 (1 x 8 x 3000 x 448: 22.4 us against 30.9; 1 x 8 x 1500 x 448, 1316
-// workgroups: 18.2 against 17.8).
-bool is_short(int64_t B, int64_t H, int64_t S, int64_t ds, bool halves) {
-  if (k1_groups(B, S, ds) >= (halves ? kMinK1Groups / 2 : kMinK1Groups)) return false;
-  const int64_t blocks = B * ((S + kBlockRows - 1) / kBlockRows);
-  return ds % 128 == 0 || H >= 16 || blocks * (ds / 64) <= 1500;
 }
 
 // Rows per scan block: S / 64 rounded up to a multiple of 16, within [16, 64],
@@ -744,6 +767,104 @@ bool is_short(int64_t B, int64_t H, int64_t S, int64_t ds, bool halves) {
 int64_t block_rows(int64_t S) {
   int64_t r = ((S + 63) / 64 + 15) / 16 * 16;
   return r < 16 ? 16 : r > 64 ? 64 : r;
+}
+
+// How one column slice of ds dims runs.
+struct Form {
+  int cw;                 // short form: dims of a column tile; 0: the long form
+  int unroll;             // heads in flight per lane
+  int planes;             // 1, or 2 head halves, each with its plane of head sums
+  const void* kernel;     // the dO pass
+};
+template <int CW, int U>
+Form short_form(bool halves, int planes) {
+  return {CW, U, planes, halves ? reinterpret_cast<const void*>(&mla_short_do<CW, U, true>)
+                                : reinterpret_cast<const void*>(&mla_short_do<CW, U, false>)};
+}
+Form long_form(bool halves, bool fits, int planes) {
+  if (halves) return {0, 1, planes, reinterpret_cast<const void*>(&mla_stream_do<1, true>)};
+  if (fits) return {0, 8, planes, reinterpret_cast<const void*>(&mla_stream_do<8, false>)};
+  return {0, 2, planes, reinterpret_cast<const void*>(&mla_stream_do<2, false>)};
+}
+
+// The form of a slice, `nexact` exact-row workgroups per batch beside it.  The lines
+// were drawn on 2581 shapes (B 1 .. 8, H 8 .. 128, S 8 .. 8192, D 64 .. 512, both types of
+// dq), each timed in every form.  us per call in a replayed graph; B x H x S x D.
+Form pick_form(int64_t B, int64_t H, int64_t S, int64_t ds, int64_t nexact, bool halves) {
+  const int64_t groups = k1_groups(B, S, ds);
+  const int64_t blocks = B * ((S + kBlockRows - 1) / kBlockRows);
+  auto tiles = [&](int64_t cw) { return blocks * (ds / cw); };
+
+  // The long form where K1's grid is large: 4 workgroups per CU, or 2 with fp32 dq,
+  // whose stores set the pass's rate (fp32, 2 x 64 x 1900 x 512: 147.9 against 154.1 in
+  // the short form; 2 x 64 x 1024 x 512: 84.6 against 85.0).  Also where only 64-dim
+  // tiles fit and few heads leave their 8 head groups one or two heads each (bf16, 1
+  // x 8 x 3000 x 448: 22.4 against 30.9; 1 x 8 x 1500 x 448: 18.2 against 17.8).
+  // U = 8 fills the chip once with 4 workgroups per CU: at 1000 to 1028 of them 26.4
+  // against 28.6 with U = 2 (1 x 8 x 4000 x 448), 109.5 against 113.9 (2 x 64 x 2048 x
+  // 512), 207.8 against 220.6 (4 x 128 x 1025 x 512); from 1050 on 117.1 with U = 2
+  // against 118.4 (2 x 64 x 2100 x 512), 121.8 against 127.3 (2200).  Multiples of 128
+  // dims meet it at 1024 workgroups only: below, the short form takes them.
+  const bool narrow_few = ds % 128 != 0 && H < 16 && tiles(64) > 1500;
+  if (groups >= (halves ? kMinK1Groups / 2 : kMinK1Groups) || narrow_few)
+    return long_form(halves, groups <= kMinK1Groups, 1);
+
+  // Many heads make a short-form workgroup's chain long and its last round costly:
+  // there the heads are halved over workgroups, each half with its plane of sums.
+  const bool fits = tiles(128) + B * nexact <= 320;   // 128-dim tiles and exact rows: one round
+  if (H >= 40) {
+    // Two planes need scan blocks of 16 rows (mla_short_scan); behind hundreds of exact
+    // rows a call of a few rows gains nothing (bf16 8 x 128 x 11 x 512 21.9, not halved 19.5).
+    const bool pairs = S <= 1024 && (S >= 32 || B * H <= 512);
+    if (ds % 128 != 0) {
+      // fp32 1 x 128 x 265 x 192 16.3 against 21.6, 2 x 128 x 197 x 192 24.7 / 33.8, 1 x 64 x 313
+      // x 192 13.3 / 14.6; past the line 1 x 64 x 281 x 448 (252 tiles) 18.9 / 18.0; 4 x 128 x 103 x
+      // 320, 39.1 / 31.8, is the one shape measured more than 8 % slower.
+      if (pairs && ((tiles(64) <= 128 && (S >= 32 || B == 1)) || (H >= 112 && tiles(64) <= 400)))
+        return short_form<64, 4>(halves, 2);
+    } else {
+      // Halved 128-dim tiles of at most one per CU: fp32 1 x 128 x 100 x 512 18.3 against
+      // 24.9, 1 x 128 x 185 23.3 / 28.9, 1 x 64 x 200 16.1 / 17.3, 1 x 64 x 246 (124 tiles) 18.0 /
+      // 17.6; past the line 1 x 64 x 300 (152) 21.0 / 17.7.  Fewer yet: 64-dim tiles, fp32 1 x
+      // 128 x 34 14.0 / 20.5, bf16 1 x 128 x 64 12.5 / 19.1.  Where the tiles and the exact rows do
+      // not fit one round, halved tiles even the rounds (not halved: 64-dim tiles, which do
+      // so too): fp32 1 x 128 x 420 x 512 41.9 / 48.8, 3 x 128 x 102 44.1 / 57.4, 2 x 64 x 300 31.2 /
+      // 36.1, bf16 2 x 64 x 300 24.9 / 26.1.  8 heads in flight where a wave has 16 heads.
+      if (pairs && tiles(64) <= 96) return short_form<64, 4>(halves, 2);
+      if (pairs && (tiles(128) <= 128 || (tiles(128) < 320 && !fits)))
+        return H >= 112 && B <= 2 ? short_form<128, 8>(halves, 2) : short_form<128, 4>(halves, 2);
+      if (ds % 256 == 0 && tiles(256) >= 320) {
+        // The long form halved, smaller workgroups than tiles that fill a second or
+        // third round badly: fp32 1 x 128 x 1300 x 512 101.6 against 126.0, 1 x 64 x 1500
+        // 64.0 / 71.3, past the line 1 x 64 x 1657 (416 tiles) 78.6 / 76.7; bf16 1 x 128 x 2400
+        // 123.6 / 140.8, 1 x 64 x 2700 80.0 / 82.4, 2 x 128 x 1100 121.3 / 128.1, but 1 x 64 x 1800
+        // (450 tiles) 60.2 / 54.7, 1 x 64 x 3400 (850) 96.7 / 93.5, 2 x 64 x 1500 (752) 84.3 / 79.4.
+        if (halves ? B <= 2 && H >= 48 && tiles(256) <= 384
+                   : tiles(256) >= 520 && (B == 1 ? H >= 64 && tiles(256) < 760
+                                                  : B == 2 && H >= 96 && tiles(256) < 640))
+          return long_form(halves, false, 2);
+        // Three batches' exact rows and wide tiles: fp32 4 x 64 x 420 x 512 70.4 against
+        // 85.9, bf16 4 x 128 x 420 92.3 / 106.4, 3 x 64 x 687 62.3 / 66.2, 4 x 64 x 850 93.7 / 103.2.
+        if (B >= 3 && H >= 64) return short_form<128, 8>(halves, pairs ? 2 : 1);
+      } else if (B >= 3 && pairs && tiles(128) >= 320) {
+        // bf16 4 x 128 x 199 x 512 52.7 against 64.1 not halved, 8 x 64 x 132 37.8 / 41.2, fp32 4 x
+        // 64 x 223 42.4 / 50.8; with two batches 2 x 128 x 457 60.0 / 57.7.
+        return short_form<128, 8>(halves, 2);
+      }
+    }
+  }
+  // The widest tile with at least 320 workgroups, whose longer contiguous pieces of a
+  // row memory serves faster; else 128 dims with all of a wave's 8 or more heads in
+  // flight where they fit one round with the exact rows, else 64 dims.  320 is a measured
+  // line, H = 64, D = 512, bf16 (B x S: the tile of this rule, the others in the order 512
+  // / 256 / 128 / 64): 1 x 300, fp32: 128: 17.9, others 43.4 / 29.5 / - / 25.1; 2 x 1024: 256: 60.0, 68.5 /
+  // - / 62.4 / 69.9; 2 x 1900: 512: 102.2, - / 116.6 / 111.5 / 121.9.  Before the short form (partial
+  // planes, block totals, scan with the exact rows): 25.6, 62.1 and 109.3.
+  if (ds % 512 == 0 && tiles(512) >= 320) return short_form<512, 4>(halves, 1);
+  if (ds % 256 == 0 && tiles(256) >= 320) return short_form<256, 4>(halves, 1);
+  if (ds % 128 == 0 && tiles(128) >= 320) return short_form<128, 4>(halves, 1);
+  if (ds % 128 == 0 && fits) return short_form<128, 8>(halves, 1);
+  return short_form<64, 4>(halves, 1);
 }
 
 // Dims of column slice `i` of D (slices of kSliceD, the last one shorter).
@@ -784,6 +905,12 @@ namespace fagq {
 namespace mla {
 namespace {
 
+int check_sizes(int64_t B, int64_t H, int64_t S, int64_t D) {
+  if (B < 0 || H < 1 || S < 1 || D < 64 || D % 64 != 0) return FAGQ_E_SHAPE;
+  if (B > 65535 || H > 65535 || H * S * D * 4 >= (1ll << 32)) return FAGQ_E_TOO_LARGE;
+  return FAGQ_OK;
+}
+
 // Argument checks shared by both entry points (everything but the workspace);
 // *need receives the workspace bytes the call uses.
 int check_args(const void* q, const void* c_kv, const void* out, const void* dout,
@@ -793,9 +920,9 @@ int check_args(const void* q, const void* c_kv, const void* out, const void* dou
   if ((dq_dtype != FAGQ_MLA_F32 && dq_dtype != FAGQ_MLA_BF16) ||
       (dc_dtype != FAGQ_MLA_F32 && dc_dtype != FAGQ_MLA_BF16))
     return FAGQ_E_FORMAT;
-  if (B < 0 || H < 1 || S < 1 || D < 64 || D % 64 != 0 || !(sm_scale == sm_scale))
-    return FAGQ_E_SHAPE;
-  if (B > 65535 || H > 65535 || H * S * D * 4 >= (1ll << 32)) return FAGQ_E_TOO_LARGE;
+  if (!(sm_scale == sm_scale)) return FAGQ_E_SHAPE;
+  const int sizes = check_sizes(B, H, S, D);
+  if (sizes != FAGQ_OK) return sizes;
   *need = workspace_bytes(B, S, D);
   if (*need < 0) return FAGQ_E_TOO_LARGE;
   if (!aligned(q, 16) || !aligned(c_kv, 16) || !aligned(out, 16) || !aligned(dout, 16) ||
@@ -839,47 +966,48 @@ int launch(const void* q, const void* c_kv, const void* out, const void* dout, c
     g.lse = lse;
     g.dq = static_cast<uint8_t*>(dq) + col * qb;   // K1's rows; the exact rows run with col = 0
     g.dc = static_cast<uint8_t*>(dc_kv) + col * cb;
+    g.nexact = sl == 0 ? (int32_t)H : 0;
+    const Form f = pick_form(B, H, S, ds, g.nexact, dq_dtype == FAGQ_MLA_F32);
+    g.planes = f.planes;
+    g.hs_plane = B * S * ds;
     g.hs = static_cast<float*>(workspace);
     g.brows = (int32_t)block_rows(S);
     g.nblk = (int32_t)((S + g.brows - 1) / g.brows);
-    g.tot = g.hs + B * S * ds;
+    g.tot = g.hs + g.planes * g.hs_plane;
     g.H = (int32_t)H;
     g.S = (int32_t)S;
     g.D = (int32_t)ds;
     g.ld = (int32_t)D;
-    g.nexact = sl == 0 ? (int32_t)H : 0;
     g.erows = (int32_t)(S < kE ? S : kE);
     g.scale = sm_scale;
     g.dq_bf16 = dq_dtype == FAGQ_MLA_BF16;
     g.dc_bf16 = dc_dtype == FAGQ_MLA_BF16;
     void* args[] = {&g};
-    const bool halves = dq_dtype == FAGQ_MLA_F32;
-    const int64_t groups = k1_groups(B, S, ds);
-    if (is_short(B, H, S, ds, halves)) {
-      const ShortTile tile = short_tile(B, S, ds, g.nexact, halves);
-      const int64_t blocks = (S + kBlockRows - 1) / kBlockRows * (ds / tile.cw);
-      const size_t join = (size_t)tile.head_groups * kBlockRows * tile.cw * 4;
+    if (f.cw != 0) {
+      const int64_t blocks = (S + kBlockRows - 1) / kBlockRows * (ds / f.cw) * f.planes;
+      const size_t join = (size_t)kShortWaves * 64 * 8 * 4;   // 8 floats of each lane
       const size_t exact = g.nexact ? exact_lds_bytes(D) : 0;
-      // nexact + blocks < 2^17 + 2^26: H S D 4 < 2^32 and D >= 64.
-      int ls = launch_kernel(tile.kernel, dim3((unsigned)(g.nexact + blocks), (unsigned)B),
+      // nexact + blocks < 2^17 + 2^27: H S D 4 < 2^32 and D >= 64.
+      int ls = launch_kernel(f.kernel, dim3((unsigned)(g.nexact + blocks), (unsigned)B),
                              dim3(64 * kShortWaves), args, join > exact ? join : exact, st);
       if (ls != FAGQ_OK) return ls;
-      ls = launch_kernel(reinterpret_cast<const void*>(&mla_short_scan),
-                         dim3((unsigned)g.nblk, (unsigned)B), dim3(kWide), args, 0, st);
+      const void* scan = f.planes == 2 ? reinterpret_cast<const void*>(&mla_short_scan<2, 2>)
+                                       : reinterpret_cast<const void*>(&mla_short_scan<1, kBlockRows>);
+      ls = launch_kernel(scan, dim3((unsigned)g.nblk, (unsigned)B), dim3(kWide), args, 0, st);
       if (ls != FAGQ_OK) return ls;
       continue;
     }
     const int rows_per_wg = kThreads / (int)(ds / 8);
-    const dim3 k1_grid((unsigned)((S + rows_per_wg - 1) / rows_per_wg), (unsigned)B);
-    const void* k1 = halves                    ? reinterpret_cast<const void*>(&mla_stream_do<1, true>)
-                     : groups <= kMinK1Groups ? reinterpret_cast<const void*>(&mla_stream_do<8, false>)
-                                              : reinterpret_cast<const void*>(&mla_stream_do<2, false>);
-    int ls = launch_kernel(k1, k1_grid, dim3(kThreads), args, 0, st);
+    const dim3 k1_grid((unsigned)((S + rows_per_wg - 1) / rows_per_wg), (unsigned)B,
+                       (unsigned)f.planes);
+    int ls = launch_kernel(f.kernel, k1_grid, dim3(kThreads), args, 0, st);
     if (ls != FAGQ_OK) return ls;
     // nblk < 2^20 and nexact + nblk < 2^17 + 2^20: nblk <= S / 16 + 1 and
     // H S D 4 < 2^32 with D >= 64.
-    ls = launch_kernel(reinterpret_cast<const void*>(&mla_block_totals),
-                       dim3((unsigned)g.nblk, (unsigned)B), dim3(kWide), args, kBlockTotalLds, st);
+    const void* totals = f.planes == 2 ? reinterpret_cast<const void*>(&mla_block_totals<2>)
+                                       : reinterpret_cast<const void*>(&mla_block_totals<1>);
+    ls = launch_kernel(totals, dim3((unsigned)g.nblk, (unsigned)B), dim3(kWide), args,
+                       kBlockTotalLds, st);
     if (ls != FAGQ_OK) return ls;
     ls = launch_kernel(reinterpret_cast<const void*>(&mla_exact_rows_suffix_scan),
                        dim3((unsigned)(g.nexact + g.nblk), (unsigned)B), dim3(kWide), args,
@@ -941,6 +1069,22 @@ FAGQ_API int fagq_mla_bwd_launch(const void* q, const void* c_kv, const void* ou
   if (B == 0) return FAGQ_OK;
   return launch(q, c_kv, out, dout, lse, dq, dc_kv, workspace, need, B, H, S, D, sm_scale,
                 dq_dtype, dc_dtype, stream);
+}
+
+FAGQ_API int fagq_mla_bwd_query_route(int64_t B, int64_t H, int64_t S, int64_t D, int dq_dtype,
+                                      int64_t slice, fagq_mla_route* route) {
+  if (!route) return FAGQ_E_NULL;
+  if (dq_dtype != FAGQ_MLA_F32 && dq_dtype != FAGQ_MLA_BF16) return FAGQ_E_FORMAT;
+  const int sizes = check_sizes(B, H, S, D);
+  if (sizes != FAGQ_OK) return sizes;
+  if (slice < 0 || slice >= (D + kSliceD - 1) / kSliceD) return FAGQ_E_SHAPE;
+  const int64_t ds = slice_dims(D, slice);
+  const Form f = pick_form(B, H, S, ds, slice == 0 ? H : 0, dq_dtype == FAGQ_MLA_F32);
+  route->dims = (int32_t)ds;
+  route->tile_dims = f.cw;
+  route->heads_in_flight = f.unroll;
+  route->head_planes = f.planes;
+  return FAGQ_OK;
 }
 
 FAGQ_API int fagq_mla_bwd_launch_noalloc(const void* q, const void* c_kv, const void* out,

@@ -55,6 +55,19 @@ FAGQ_API int fagq_gemm_launch_mapped(const void* a_q, const void* a_scale, const
                                      int64_t K, int a_scale_format, int a_scale_layout,
                                      int b_scale_format, int block_n, void* stream);
 
+/* How fagq_mla_bwd_launch (fagq_mla.h) runs column slice `slice` (of
+ * FAGQ_MLA_SLICE_D dims) of a shape.  Never touches the device.  The arguments'
+ * limits are fagq_mla_bwd_launch's (FAGQ_E_SHAPE, FAGQ_E_TOO_LARGE, FAGQ_E_FORMAT). */
+typedef struct fagq_mla_route {
+  int32_t dims;            /* columns of the slice */
+  int32_t tile_dims;       /* short form (two launches): columns of a tile; 0: the long form */
+  int32_t heads_in_flight; /* per lane of the dO pass */
+  int32_t head_planes;     /* 1, or 2: the heads halved over workgroups */
+} fagq_mla_route;
+
+FAGQ_API int fagq_mla_bwd_query_route(int64_t B, int64_t H, int64_t S, int64_t D, int dq_dtype,
+                                      int64_t slice, fagq_mla_route* route);
+
 /* Encodes n fp32 values (n % 8 == 0, 16-byte aligned) with the operator's
  * device encoder: one byte per value.  clamp = 1 applies the reference's
  * clamp to [-QMAX, QMAX] first; clamp = 0 passes the values unclamped, as the
