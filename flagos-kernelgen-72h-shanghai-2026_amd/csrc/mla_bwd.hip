@@ -744,7 +744,6 @@ bool overlap(const void* a, int64_t na, const void* b, int64_t nb) {
 }
 
 constexpr int kMinK1Groups = 1024;        // K1 workgroups wanted (4 per CU)
-constexpr int kMaxHeadSplit = 8;
 
 // K1's workgroups for a column slice of D dims.
 int64_t k1_groups(int64_t B, int64_t S, int64_t D) {
@@ -752,13 +751,10 @@ int64_t k1_groups(int64_t B, int64_t S, int64_t D) {
   return ((S + rows_per_wg - 1) / rows_per_wg) * B;
 }
 
-// Planes of head sums the workspace is sized for.  The kernels use one or two;
-// the size that callers were told for a shape does not change.
+// Planes of head sums a slice of D dims may need, whatever its heads and types
+// (pick_form halves the heads below kMinK1Groups only).
 int64_t workspace_planes(int64_t B, int64_t S, int64_t D) {
-  if (D < 64) return 1;
-  int64_t sp = 1;
-  while (k1_groups(B, S, D) * sp < kMinK1Groups && sp < kMaxHeadSplit) sp *= 2;
-  return sp;
+  return D >= 64 && k1_groups(B, S, D) < kMinK1Groups ? 2 : 1;
 }
 
 // Rows per scan block: S / 64 rounded up to a multiple of 16, within [16, 64],

@@ -38,9 +38,9 @@ extern "C" {
 
 enum fagq_mla_dtype { FAGQ_MLA_F32 = 0, FAGQ_MLA_BF16 = 1 };
 
-/* Workspace bytes fagq_mla_bwd_launch needs for (B, S, D): room for fp32 head
- * sums [G, B, S, W] (G = 1 when the row grid fills the GPU, else up to 8: the
- * kernels use one) and the scan's block totals [B, nblk, W] (blocks of 16-64
+/* Workspace bytes fagq_mla_bwd_launch needs for (B, S, D): fp32 head sums
+ * [G, B, S, W] (G = 1 when the row grid fills the GPU, else 2, one for each half
+ * of many heads) and the scan's block totals [B, nblk, W] (blocks of 16-64
  * rows), W = min(D, FAGQ_MLA_SLICE_D).  Returns -1 for a negative or
  * overflowing size. */
 FAGQ_API int64_t fagq_mla_bwd_workspace_bytes(int64_t B, int64_t S, int64_t D);

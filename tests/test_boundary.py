@@ -562,9 +562,8 @@ def test_mla_validation(lib, kw, status):
 def test_mla_workspace_size(lib):
     # head sums [B, S, D] plus the totals of 64-row blocks
     assert lib.fagq_mla_bwd_workspace_bytes(2, 4096, 512) == 2 * (4096 + 64) * 512 * 4
-    # small grids split the heads into up to 8 groups, one partial plane each;
-    # 16-row blocks
-    assert lib.fagq_mla_bwd_workspace_bytes(1, 65, 64) == (8 * 65 + 5) * 64 * 4
+    # small grids may halve the heads, one partial plane each; 16-row blocks
+    assert lib.fagq_mla_bwd_workspace_bytes(1, 65, 64) == (2 * 65 + 5) * 64 * 4
     assert lib.fagq_mla_bwd_workspace_bytes(-1, 1, 64) == -1
     # D above 512 runs in 512-wide column slices: the workspace holds one slice
     assert lib.fagq_mla_bwd_workspace_bytes(2, 4096, 1024) == 2 * (4096 + 64) * 512 * 4

@@ -82,3 +82,29 @@ def test_random_long(pkg, gpu, seed):
     S = rows * -(-(512 if grad == F32 else 1024) // B) + rng.randint(0, 2 * rows)
     assert forms(B, H, S, D, grad)[0][0] == 0
     case(pkg, gpu, B, H, S, D, grad, rng.choice([None, F32, BF16]), seed=seed)
+
+
+@pytest.mark.parametrize("B,H,S,D,grad", [(1, 128, 34, 512, F32), (1, 128, 150, 512, BF16), (1, 4, 40, 576, F32),
+                                          (1, 48, 1024, 64, BF16), (1, 48, 1283, 512, F32), (1, 3, 4096, 512, BF16),
+                                          (1, 3, 4100, 576, BF16), (2, 49, 37, 192, F32)])
+def test_workspace_of_the_told_size(pkg, gpu, B, H, S, D, grad):
+    """No form writes past the workspace bytes that a caller is told, and its results do
+    not depend on what they held."""
+    from fagq_mi355x import mla_bwd
+    from fagq_mi355x.workloads import MlaWorkload, make_mla_inputs
+    from tests.gpu_util import note
+    note(f"mla workspace B{B} H{H} S{S} D{D} {grad}")
+    w = MlaWorkload("t", B, H, S, D, grad, seed=S)
+    q, c, out, do, lse = make_mla_inputs(w, device=gpu)
+    need = mla_bwd.workspace_bytes(B, S, D)
+    got = []
+    for fill in (0, 0xFF):                                  # 0xFF: NaN as fp32
+        buf = torch.full((need + 8192,), 0xA5, dtype=torch.uint8, device=gpu)
+        buf[:need] = fill
+        dq, dc = torch.empty_like(q, dtype=grad), torch.empty_like(c, dtype=grad)
+        pkg.mla_bwd_nope_dkdv(q, c, out, do, lse, dq, dc, w.sm_scale, workspace=buf[:need])
+        torch.cuda.synchronize()
+        assert bool((buf[need:] == 0xA5).all())
+        got.append((dq, dc))
+    for a, b in zip(*got):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
