@@ -65,10 +65,12 @@ def test_quantizer_graph_replays_match_eager(pkg, gpu, M, D, qdt, col, ue8m0):
 
 
 @pytest.mark.parametrize("S,gdt", [
-    (512, torch.bfloat16),       # 128 row workgroups x 8 head groups: the wide K1
+    (512, torch.bfloat16),       # the short form
+    (4096, torch.bfloat16),      # the long form, 1024 row workgroups: 8 heads in flight
+    (4100, torch.bfloat16),      # 1025 row workgroups: 2 heads in flight
     (8192, torch.float32)])      # 2048 row workgroups: the one-head-in-flight fp32 K1
 def test_mla_noalloc_graph_replays_match_eager(pkg, gpu, S, gdt):
-    """fagq_mla_bwd_launch_noalloc (three kernels, the library's own workspace)
+    """fagq_mla_bwd_launch_noalloc (two or three kernels, the library's own workspace)
     captured once and replayed with new dO between replays, against the
     caller-workspace entry point run eagerly."""
     from fagq_mi355x import _lib

@@ -84,9 +84,9 @@ def case(pkg, dev, B, H, S, D, grad_dtype, dc_dtype=None, seed=0):
         f"{label}: dc off by {float((err - tol).max())} over tolerance"
 
 
-# Short sequences split the heads into several partial head-sum planes and
-# their scan blocks into column slices (S = 256, 512); 769, 1024, 1025 and 2048
-# cover block counts that do not divide the rows evenly and fewer planes.
+# All run in the short form, in column tiles of 64 to 256 dims (test_gpu_mla_forms.py
+# has the long form, and more of the halved heads); 769, 1024, 1025 and 2048 rows cover block
+# counts that do not divide the rows evenly.
 @pytest.mark.parametrize("B,H,S,D", [(1, 4, 64, 512), (2, 3, 100, 64), (1, 2, 10, 128),
                                      (1, 8, 257, 256), (2, 64, 256, 512), (2, 64, 512, 512),
                                      (1, 1, 1, 64), (1, 4, 1024, 128), (1, 4, 1025, 128),
@@ -100,9 +100,9 @@ def test_mla_matches_oracle(pkg, gpu, B, H, S, D, grad):
                                      (1, 7, 129, 384)])
 @pytest.mark.parametrize("dq_dtype", [torch.bfloat16, torch.float32])
 def test_mla_uneven_head_groups(pkg, gpu, B, H, S, D, dq_dtype):
-    # short sequences split the heads into 3, 5, 7 and 4 groups of partial
-    # head sums; D not a power of two leaves some scan threads idle, and with
-    # fp32 dq the dO pass splits each row into two halves of D / 2
+    # 5, 9, 13 and 7 heads over the 8 (384 dims: 4) head groups of a tile leave
+    # groups short or empty; D not a power of two leaves some scan threads idle,
+    # and with fp32 dq a lane takes half of its elements from each half of the tile
     case(pkg, gpu, B, H, S, D, dq_dtype, torch.float32, seed=B + H + S)
 
 
@@ -112,8 +112,8 @@ def test_mla_uneven_head_groups(pkg, gpu, B, H, S, D, dq_dtype):
 def test_mla_column_slices(pkg, gpu, B, H, S, D, dq_dtype):
     # D above 512 runs in 512-wide column slices (the last one 64, 512, 128,
     # 128 and 512 wide): the exact rows stage their rows in chunks and the
-    # other kernels run once per slice; the last case's slices each split the
-    # heads into 8 partial planes and the block totals into 4 column slices
+    # other kernels run once per slice, here all in the short form; the last
+    # case's slices pick different ones, as only the first has exact rows beside it
     case(pkg, gpu, B, H, S, D, dq_dtype, seed=D + S)
 
 

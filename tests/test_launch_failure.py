@@ -70,12 +70,17 @@ def test_every_launching_entry_point_reports_it(seam):
     st = seam.fagq_gemm_launch(fake(0), fake(1), fake(2), fake(3), fake(4), 256, 256, 1024, 0, 1, 0,
                                None)
     assert st == -HIP_ERROR_LAUNCH_FAILURE
-    # MLA backward: the first of its three launches fails and the call stops there.
+    # MLA backward: the first of its launches (two in the short form, three in the
+    # long one) fails and the call stops there.
     B, H, S, D = 1, 4, 256, 512
     need = seam.fagq_mla_bwd_workspace_bytes(B, S, D)
     assert need > 0
     st = seam.fagq_mla_bwd_launch(fake(0), fake(1), fake(2), fake(3), fake(4), fake(5), fake(6),
                                   fake(7), need, B, H, S, D, 0.05, 1, 1, None)
+    assert st == -HIP_ERROR_LAUNCH_FAILURE
+    need = seam.fagq_mla_bwd_workspace_bytes(B, 8192, D)
+    st = seam.fagq_mla_bwd_launch(fake(0), fake(1), fake(2), fake(3), fake(4), fake(5), fake(6),
+                                  fake(7), need, B, H, 8192, D, 0.05, 1, 1, None)
     assert st == -HIP_ERROR_LAUNCH_FAILURE
     # The allocation-free form looks up its array's device address first; on
     # a host without a GPU that runtime call's error is what comes back.
