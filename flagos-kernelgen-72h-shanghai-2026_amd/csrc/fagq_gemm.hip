@@ -579,12 +579,18 @@ using Ring96x96 = Ring<3, 3, 2, 2, 3>;       // two workgroups per CU
 // slower in a small tile.
 constexpr double kPP256C = 13.0, kPP256T = 1.368, kPP192C = 10.5, kPP192T = 0.86;
 constexpr int64_t kSmallMinBlocks = 4;       // k-blocks: the fits' range ends at K = 512
-constexpr int64_t kSmallMaxK = 1 << 16;      // row offsets of 192 rows stay far below 2^31
+// Row offsets of 192 rows stay far below 2^31.  Past K = 7168 the lines are extrapolated:
+// of 100 shapes with K 7424 .. 65536 none was slower than in the 256-row tiles (geometric
+// mean 0.10 of their time), and of 8 timed in every tile each took the fastest or one
+// within 5 % (256 x 4096 x 16384: 64 x 64, 42 us, 256-row tiles 147; 500 x 2048 x 65536: 64 x
+// 64, 152, others 187 .. 593).
+constexpr int64_t kSmallMaxK = 1 << 16;
 constexpr int64_t kSmallMaxRows = 1 << 16;   // M and N of a forced small tile: a call's own reach
 
 // The small tile for a product, or kNoSmall where the 256-row tiles stay:
-// where these fill the chip once and more, outside the fits' range of K, and
-// unless a small tile is 5 % faster by the model (the model's own error).
+// where these fill the chip once and more, below 4 k-blocks (where nothing was
+// fitted) and past K = 2^16, and unless a small tile is 5 % faster by the model (the
+// model's own error).
 int pick_small(int64_t M, int64_t N, int64_t K, int pp_bn) {
   const int64_t nk = K / kBK;
   if (nk < kSmallMinBlocks || K > kSmallMaxK ||

@@ -69,8 +69,8 @@ __global__ void __launch_bounds__(64 * W) fagq_gemm_waves_kernel(const GArgs g) 
   auto load = [&](Block& x, int i) {
     const int kb = wave + W * i;
     const bool ok = kb < g.kblocks;
-    // 2^31 and up: past every operand (64 K bytes at most, K <= 2^16) and scale
-    // array (32 MB at most: one round of 256-row tiles has 2^16 rows).
+    // 2^31 and up: past every operand (4 MiB at most: 64 rows, K <= 2^16) and scale
+    // array (128 MiB at most: 2^16 rows, 512 k-blocks of 4 bytes).
     const uint32_t far = 0x80000000u;
     const uint32_t ko = (uint32_t)__builtin_amdgcn_readfirstlane(
         (int)(ok ? (uint32_t)kb * (uint32_t)kBK : far));
@@ -175,7 +175,10 @@ __global__ void __launch_bounds__(64 * W) fagq_gemm_waves_kernel(const GArgs g) 
 // (64 x 64), 512 x 4096 x 7168 55.7 -> 23.0 (128 x 64), 1000 x 2112 x 7168 56.4
 // -> 25.5 (96 x 96; 128 x 128: 30.2), 1500 x 4096 x 7168 57.3 -> 46.4 (192 x 128).
 // The 96 x 96 tile with 6 waves: 24.8 .. 27.7 there, but 46 against 41 us at 2048 x 2112 x
-// 7168, where two workgroups share a CU; 4 waves with 4 or 6 stages 29.5 and 32.0.
+// 7168, where two workgroups share a CU.  4 waves with 4 or 6 stages took 29.5 and 32.0,
+// which says nothing of the depth: with LDS for one workgroup per CU only, the launch
+// bounds allow 512 registers, the compiler keeps the 36 accumulators in AGPRs, and each
+// k-block then moves them to VGPRs and back (51 v_accvgpr moves a k-block, none with 3 stages).
 template <int TM_, int TN_, int WM_, int WN_, int S_>
 struct Ring {
   static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, S = S_;

@@ -20,8 +20,11 @@
  * then fp32 across blocks: in block order, or for small products (tiles of
  * 16 x 16 to 32 x 64, fagq_gemm_query_route) in eight interleaved partial sums
  * that are then added.  The order depends on the shape alone, so equal calls
- * give equal bits.  With both scales UE8M0 the scales are applied by the matrix
- * core itself (exact powers of two).
+ * give equal bits; it depends on M too, so one row's bits can differ between
+ * calls with other numbers of rows (both within the same error bound).
+ * fagq_gemm_launch_mapped (fagq_diag.h) with block_n 192 or 256 keeps block order
+ * at any M.  With both scales UE8M0 the scales are applied by the matrix core
+ * itself (exact powers of two).
  *
  * Same conventions as fagq.h: device pointers, stream-ordered, no allocation,
  * no synchronization; returns 0, a FAGQ_E_* code (> 0) or -hipError_t.
