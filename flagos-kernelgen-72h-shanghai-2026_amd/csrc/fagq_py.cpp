@@ -35,6 +35,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <vector>
 
 #include "fagq.h"
 #include "fagq_dsa.h"
@@ -306,11 +307,12 @@ PyObject* quant(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int64_t groups = D / G;
 
   // The list is the caller's to change once the GIL is released: its tensors are held.
-  at::Tensor held[FAGQ_MAX_PARTS];
+  std::vector<at::Tensor> held;
+  if (multi) held.reserve(n);
   const void* ptrs[FAGQ_MAX_PARTS];
   for (Py_ssize_t i = 0; i < n; ++i) {
     const at::Tensor& t = THPVariable_Unpack(xs[i]);
-    if (multi) held[i] = t;
+    if (multi) held.push_back(t);
     ptrs[i] = t.data_ptr();
   }
   const void* const rp = residual.data_ptr();

@@ -149,6 +149,10 @@ GEMM_CONFIGS = {
     "gemm_dsv3_ue8m0_16384x4096x7168": GemmWorkload("gemm_dsv3_ue8m0_16384x4096x7168", 16384,
                                                     4096, 7168, "ue8m0", "ue8m0"),
     "gemm_qkva_16384x2112x7168": GemmWorkload("gemm_qkva_16384x2112x7168", 16384, 2112, 7168),
+    # small products: a decode step of 32 sequences, and a ragged chunk's q_a + kv_a projection
+    "gemm_decode_32x4096x7168": GemmWorkload("gemm_decode_32x4096x7168", 32, 4096, 7168),
+    "gemm_chunk_ue8m0_1000x2112x7168": GemmWorkload("gemm_chunk_ue8m0_1000x2112x7168", 1000, 2112,
+                                                    7168, "ue8m0", "ue8m0"),
 }
 
 
