@@ -784,7 +784,7 @@ Form long_form(bool halves, bool fits, int planes) {
 }
 
 // The form of a slice, `nexact` exact-row workgroups per batch beside it.  The lines
-// were drawn on 2581 shapes (B 1 .. 8, H 8 .. 128, S 8 .. 8192, D 64 .. 512, both types of
+// were drawn on 2520 shapes (B 1 .. 8, H 8 .. 128, S 8 .. 8192, D 64 .. 512, both types of
 // dq), each timed in every form.  us per call in a replayed graph; B x H x S x D.
 Form pick_form(int64_t B, int64_t H, int64_t S, int64_t ds, int64_t nexact, bool halves) {
   const int64_t groups = k1_groups(B, S, ds);
